@@ -104,7 +104,8 @@ int rdv_mlp_pack(const rdv_mlp_desc* desc, const float* const* weights,
 /* y[n, dims[L]] = chain(x[n, in_features]) for fp32 row-major x and y.  Every
  * all-LinearFast chain runs on the fp16 matrix cores (a compile-time kernel for
  * the benchmark shapes, a runtime-shaped one for the rest); chains with an
- * exact fp32 Linear layer run on the vector ALUs.
+ * exact fp32 Linear layer run on the fp32 matrix cores, which chain fused
+ * multiply-adds in ascending k as Linear does.
  * Replaces Map.__call__ -> dispatch(MapEvaluator) over a chain of
  * LinearFast / Linear / ReLU maps (src/rdv/maths/__init__.py:1451-1487,
  * src/rdv/shaders/maps/map_evaluator.h:1-5, composite.h:8-12).
@@ -130,7 +131,8 @@ int64_t rdv_mlp_unpacked_workspace_bytes(const rdv_mlp_desc* desc);
  * exact-fp32 launch of a partial last 32-row group, which reads W directly;
  * no workspace.  Other chains: packed into `workspace` (256-byte aligned,
  * rdv_mlp_unpacked_workspace_bytes bytes; RDV_ERR_WORKSPACE when smaller) by
- * one pack launch, then rdv_mlp_forward.  Same results as rdv_mlp_pack +
+ * one pack launch, then rdv_mlp_forward (chains with an exact fp32 layer ask
+ * for the same workspace but read the parameters directly).  Same results as rdv_mlp_pack +
  * rdv_mlp_forward.  Replaces Map.__call__ -> dispatch(MapEvaluator), whose
  * LinearFast reads the weights through their buffer pointers at every dispatch
  * (src/rdv/maths/__init__.py:1451-1487, src/rdv/shaders/maps/linear_fast.h:39-60). */

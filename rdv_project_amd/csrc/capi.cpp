@@ -60,8 +60,7 @@ int launch_fused_entry_direct(const FusedEntry* e, const rdv_mlp_desc& d, const 
 bool direct_fused_ok(const FusedEntry* e, const rdv_mlp_desc& d);
 int launch_mlp_pack(const rdv_mlp_desc& d, const MlpLayout& lay, const float* const* W, const float* const* b,
                     void* packed, hipStream_t stream);
-int prepare_chain_f32(const rdv_mlp_desc& d);
-const char* chain_f32_name(const rdv_mlp_desc& d, const MlpLayout& lay);
+const char* chain_f32_name(const MlpLayout& lay);
 int64_t winograd_weight_bytes(int cin, int cout);
 int launch_winograd_transform_weight(const void* w, int w_layout, int w_dtype, int cin, int cout, void* U,
                                      hipStream_t stream);
@@ -228,6 +227,19 @@ int rdv_mlp_pack(const rdv_mlp_desc* desc, const float* const* weights, const fl
   return launch_mlp_pack(*desc, lay, weights, biases, packed, static_cast<hipStream_t>(stream));
 }
 
+// n rows of a chain with an exact-fp32 layer.  A partial last group of 32 rows
+// evaluates every layer in exact fp32 (tail_f32): a launch of its own, unless
+// no layer would be evaluated otherwise (Linear layers only).
+static int chain_f32_rows(const rdv_mlp_desc& d, const MlpLayout& lay, const void* packed, const float* x, float* y,
+                          int64_t n, bool tail_f32, hipStream_t s, const DirectWeights* dw) {
+  bool f16 = false;
+  for (int i = 0; i < d.n_layers; ++i) f16 = f16 || d.prec[i] == RDV_PREC_F16;
+  const int64_t n_full = f16 && tail_f32 ? (n / 32) * 32 : n;
+  const int rc = launch_mlp_chain_f32(d, lay, packed, x, y, 0, n_full, false, s, dw);
+  if (rc != RDV_OK || n == n_full) return rc;
+  return launch_mlp_chain_f32(d, lay, packed, x, y, n_full, n - n_full, true, s, dw);
+}
+
 static int mlp_forward_impl(const rdv_mlp_desc* desc, const void* packed, const float* x, float* y, int64_t n,
                             void* stream, bool tail_f32) {
   MlpLayout lay;
@@ -237,22 +249,14 @@ static int mlp_forward_impl(const rdv_mlp_desc* desc, const void* packed, const 
   if (n == 0) return RDV_OK;
   if (!packed || !x || !y) return fail(RDV_ERR_INVALID, "rdv_mlp_forward: NULL pointer argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const FusedEntry* e = find_fused(*desc, lay);
+  if (!e && !generic_f16_supported(*desc)) return chain_f32_rows(*desc, lay, packed, x, y, n, tail_f32, s, nullptr);
   const int64_t n_full = tail_f32 ? (n / 32) * 32 : n;
   const int64_t n_tail = n - n_full;
-  const FusedEntry* e = find_fused(*desc, lay);
-  if (e) {
-    rc = launch_fused_entry(e, *desc, lay, packed, x, y, n_full, s);
-  } else if (generic_f16_supported(*desc)) {
-    rc = launch_mlp_generic_f16(*desc, lay, packed, x, y, n_full, s);
-  } else {
-    rc = prepare_chain_f32(*desc);
-    if (rc == RDV_OK) rc = launch_mlp_chain_f32(*desc, lay, packed, x, y, 0, n_full, false, s);
-  }
+  rc = e ? launch_fused_entry(e, *desc, lay, packed, x, y, n_full, s)
+         : launch_mlp_generic_f16(*desc, lay, packed, x, y, n_full, s);
   if (rc != RDV_OK) return rc;
-  if (n_tail > 0) {
-    rc = prepare_chain_f32(*desc);
-    if (rc == RDV_OK) rc = launch_mlp_chain_f32(*desc, lay, packed, x, y, n_full, n_tail, true, s);
-  }
+  if (n_tail > 0) rc = launch_mlp_chain_f32(*desc, lay, packed, x, y, n_full, n_tail, true, s);
   return rc;
 }
 
@@ -292,6 +296,8 @@ int rdv_mlp_forward_unpacked(const rdv_mlp_desc* desc, const float* const* weigh
       return fail(RDV_ERR_WORKSPACE, "workspace of " + std::to_string(workspace_bytes) + " bytes; this chain needs " +
                                          std::to_string(lay.total_bytes));
     if (reinterpret_cast<uintptr_t>(workspace) % 256) return fail(RDV_ERR_INVALID, "workspace must be 256-byte aligned");
+    if (e == nullptr && !generic_f16_supported(*desc))  // read from the rows themselves: no pack launch
+      return chain_f32_rows(*desc, lay, nullptr, x, y, n, true, s, &dw);
     rc = launch_mlp_pack(*desc, lay, dw.W, dw.b, workspace, s);
     if (rc != RDV_OK) return rc;
     return mlp_forward_impl(desc, workspace, x, y, n, stream, true);
@@ -300,8 +306,7 @@ int rdv_mlp_forward_unpacked(const rdv_mlp_desc* desc, const float* const* weigh
   rc = launch_fused_entry_direct(e, *desc, lay, dw, x, y, n_full, s);
   if (rc != RDV_OK) return rc;
   if (n > n_full) {
-    rc = prepare_chain_f32(*desc);
-    if (rc == RDV_OK) rc = launch_mlp_chain_f32(*desc, lay, nullptr, x, y, n_full, n - n_full, true, s, &dw);
+    rc = launch_mlp_chain_f32(*desc, lay, nullptr, x, y, n_full, n - n_full, true, s, &dw);
   }
   return rc;
 }
@@ -727,7 +732,7 @@ const char* rdv_mlp_kernel_name(const rdv_mlp_desc* desc) {
   if (check_mlp(desc, &lay) != RDV_OK) return "";
   const FusedEntry* e = find_fused(*desc, lay);
   if (e) return fused_name(e);
-  return generic_f16_supported(*desc) ? generic_f16_name(*desc, lay) : chain_f32_name(*desc, lay);
+  return generic_f16_supported(*desc) ? generic_f16_name(*desc, lay) : chain_f32_name(lay);
 }
 
 }  // extern "C"

@@ -216,6 +216,36 @@ def test_f32_chain_register_kernel_equals_row_kernel(dims, precs, enc):
     assert _lib.load().rdv_mlp_kernel_name(CH.plan_chain(m, d_in).desc).decode() == "mlp_chain_f32_reg_kernel"
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 31, 144, 9000])  # 16-row tiles: one, part of one, more than a wave takes
+@pytest.mark.parametrize("dims,precs", [
+    ([1, 1], ["f32"]), ([4, 16, 16], ["f32"] * 2), ([15, 17, 5], ["f32"] * 2),   # tile edges
+    ([64, 64, 64, 1], ["f32"] * 3), ([33, 63, 49, 16], ["f32", "f16", "f32"]),    # straight-line and branching layers
+    ([3] + [64] * 11 + [2], ["f32"] * 12),                                        # parameters past the LDS: read from rows
+    ([65, 128, 250, 256, 3], ["f32"] * 4),                                        # the wide kernel, some layers from rows
+])
+def test_f32_chain_edges(dims, precs, n):
+    """Exact-fp32 chains at the edges of their 16-wide tiles, against float64:
+    layer by layer each output is an fp32 FMA chain over k inputs, off by at
+    most gamma(k + 2) of the sum of its magnitudes; the bound is carried through
+    the layers (ReLU does not grow it).  LinearFast layers round their inputs
+    and weights to fp16 (2^-11 relative each) first."""
+    g = WL.gen(57)
+    layers = [((torch.rand(dims[i + 1], dims[i], generator=g) * 2 - 1) / dims[i] ** 0.5 * 1.7,
+               torch.rand(dims[i + 1], generator=g) * 0.2 - 0.1) for i in range(len(dims) - 1)]
+    acts = ["relu"] * (len(dims) - 2) + ["none"]
+    x = torch.rand(n, dims[0], generator=g) * 2 - 1
+    y = _chain(layers, acts, f16=[p == "f16" for p in precs])(x.cuda()).as_tensor("torch").cpu().double()
+    u, v, e = 2.0 ** -24, x.double(), torch.zeros(n, dims[0], dtype=torch.float64)
+    for i, (w, b) in enumerate(layers):
+        w, k = w.double(), dims[i] + 2
+        r = k * u / (1 - k * u) + (2.01 * 2.0 ** -11 if precs[i] == "f16" else 0.0)
+        e = e @ w.abs().t() * (1 + r) + r * (v.abs() @ w.abs().t() + b.double().abs())
+        v = v @ w.t() + b.double()
+        if acts[i] == "relu":
+            v = v.clamp_min(0.0)
+    assert bool(((y - v).abs() <= e).all()), float(((y - v).abs() / e).max())
+
+
 @pytest.mark.parametrize("acts", [
     ["softplus", "relu", "none"],       # a transcendental hidden activation
     ["relu", "none", "sigmoid"],        # a linear hidden layer, sigmoid head
