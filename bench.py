@@ -423,7 +423,7 @@ def bench_tensor_ops(steps, warmup):
             "hbm_peak_pct": round(100 * nbytes / (ev * 1e-3) / 1e9 / PEAK_HBM_GBS, 2),
             "TFLOP_s": round(2.0 * n * inf * outf / (ev * 1e-3) / 1e12, 1),
             "bytes_per_call": nbytes,
-            "kernel": "linear_op_kernel<true, 2, 4>",
+            "kernel": "linear_gemm_kernel<fp16>",
         },
         "ReLUTensorOp": {
             "workload": "4,194,304 x 128 fp32",

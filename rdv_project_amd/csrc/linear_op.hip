@@ -14,27 +14,7 @@
 // at dispatch, like Small and Mine), fp16 [out, in] (Simple's pre-cast copy) or
 // fp16 [out/16][in/16][16 k][16 n] tiles (Fast's pre-tiled copy, nn.py:472-490).
 //
-// MI355X mapping.  The op is streaming: at in = out = 128 it does 32 flops per
-// HBM byte against a ridge of ~300, so the bound is HBM and the design goal is
-// to touch every x and y byte once with wide accesses while the whole weight
-// block sits in LDS.  Each workgroup (4 waves) owns one block of <= 128 outputs
-// for the whole run: it stages that block of W (and of the bias) into LDS once,
-// in MFMA-fragment order, then walks row tiles with a grid stride and no further
-// barrier.  A wave computes D^T = W x^T for 16-row subtiles:
-//   fp16: v_mfma_f32_16x16x32_f16, A = W[16 out][32 k], B = x^T[32 k][16 rows];
-//         lane (r = l%16, q = l/16) loads x[r][8q..8q+7] as two 16-byte loads.
-//   fp32: v_mfma_f32_16x16x4f32 over 16-k groups; lane (r, q) loads x[r][4q..4q+3]
-//         once and feeds one element to each of 4 MFMAs (MFMA k index q stands
-//         for k = 4q + s in step s; W fragments are staged in the same order).
-//   D[out 4q+j][row r] leaves each lane with 4 consecutive outputs of one row:
-//   one 16-byte store per (subtile, out tile).  Loads and stores are ordinary
-//   (cached): each instruction covers only half of every 128-byte line it
-//   touches, and with non-temporal hints the halves reach HBM separately
-//   (measured: 20% more bytes written and 16% lower throughput at 128 -> 128).
-// The next tile's x loads are issued right after the current tile's loads have
-// been converted, so they stream under the MFMAs and stores.  When in exceeds
-// one LDS pass (256 fp16 / 128 fp32 columns) the weight is restaged per pass and
-// per tile instead (a plain tiled GEMM).
+// linear_gemm_kernel (below) serves every shape; relu_op_kernel streams.
 #include <algorithm>
 
 #include "rdv_common.h"
@@ -43,40 +23,6 @@ namespace rdv {
 
 namespace {
 
-constexpr int kLoThreads = 256;
-constexpr int kLoWaves = kLoThreads / 64;
-constexpr int kLoMaxOb = 128;  // outputs per workgroup block
-
-struct LinearOpArgs {
-  const float* x;     // [rows, in]
-  const void* w;      // weight (wkind)
-  const float* bias;  // [out]
-  float* y;           // [rows, out]
-  int64_t rows;
-  int64_t tasks;      // row tiles of kLoWaves * 16 * RT rows
-  int in, out;
-  int wkind;          // RDV_WKIND_*
-  int relu;
-  int kp;             // columns of x per LDS pass (multiple of the k step)
-  int passes;         // ceil(in / kp)
-  int ob;             // outputs per block (multiple of 16)
-  int n_ob;           // ceil(out / ob)
-};
-
-// One k chunk of one lane: F16 -> 8 columns (two float4), F32 -> 4 columns.
-template <bool F16>
-struct LoPolicy;
-template <>
-struct LoPolicy<true> {
-  static constexpr int kStep = 32;  // columns per chunk
-  static constexpr int kVec = 2;    // float4 loads per lane per chunk
-};
-template <>
-struct LoPolicy<false> {
-  static constexpr int kStep = 16;
-  static constexpr int kVec = 1;
-};
-
 __device__ __forceinline__ half8 to_half8(f32x4 a, f32x4 b) {
   half8 h;
   h[0] = half_t(a[0]); h[1] = half_t(a[1]); h[2] = half_t(a[2]); h[3] = half_t(a[3]);
@@ -84,157 +30,241 @@ __device__ __forceinline__ half8 to_half8(f32x4 a, f32x4 b) {
   return h;
 }
 
-// Stages outputs [o0, o0 + ob) x columns [k0, k0 + kp) of W into LDS in fragment
-// order: slot ((t * nkc + c) * 64 + lane) holds 16 bytes, W[o0 + 16t + lane%16]
-// [k0 + c*kStep + (lane/16)*(kStep/4) ...] as 8 halves (fp16) or 4 floats (fp32).
-// Rows past `out` and columns past `in` are zero.  Also stages the bias block.
-template <bool F16>
-__device__ void stage_weight(const LinearOpArgs& a, int o0, int k0, int nkc, f32x4* sw, float* sb) {
-  using P = LoPolicy<F16>;
-  const int nt = a.ob / 16;
-  const int slots = nt * nkc * 64;
-  for (int s = threadIdx.x; s < slots; s += kLoThreads) {
-    const int t = s / (nkc * 64);
-    const int rem = s - t * (nkc * 64);
-    const int c = rem >> 6;
-    const int ln = rem & 63;
-    const int o = o0 + 16 * t + (ln & 15);
-    const int k = k0 + c * P::kStep + (ln >> 4) * (P::kStep / 4);
-    const bool ok = o < a.out && k < a.in;
-    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (ok) {
-      if constexpr (F16) {
-        half8 h;
-        if (a.wkind == RDV_WKIND_F32) {
-          const f32x4* src = reinterpret_cast<const f32x4*>(static_cast<const float*>(a.w) + int64_t(o) * a.in + k);
-          h = to_half8(src[0], src[1]);
-        } else if (a.wkind == RDV_WKIND_F16) {
-          h = *reinterpret_cast<const half8*>(static_cast<const half_t*>(a.w) + int64_t(o) * a.in + k);
-        } else {  // fp16 tiles [out/16][in/16][16 k][16 n]
-          const half_t* wt = static_cast<const half_t*>(a.w);
-          const int64_t base = (int64_t(o >> 4) * (a.in >> 4) + (k >> 4)) * 256 + (o & 15);
+// ---------------------------------------------------------------- linear ops
+// A tiled product.  A block of NW waves (2 across the rows, NW / 2 across the
+// outputs) computes BM rows x BN outputs; per K step of 64 (fp16) or 32 (fp32)
+// columns it stages both operands' tiles in LDS as MFMA fragments, double
+// buffered: the next step's global loads are in flight during this step's MFMAs,
+// and one barrier per step suffices.  D^T = W x^T, so a lane ends with 4
+// consecutive outputs of one row: one cached 16-byte store per 16 x 16 tile.
+//   fp16: v_mfma_f32_16x16x32_f16 over chunks of 32 columns, x rounded on the way
+//         into LDS; fp32: v_mfma_f32_16x16x4f32 over chunks of 16 (quarter q holds
+//         columns 4q + s in step s).  Bias first, chunks ascending.
+// TILED: the weight is the fp16 tile layout [out/16][in/16][16 k][16 n].  Its
+// tiles go from global memory straight into LDS (global_load_lds_dwordx4) and
+// the fragments' transpose is done by ds_read_b64_tr_b16, which hands lane i of 16
+// column i of a 4 x 16 block (through registers it is eight 2-byte loads per piece).
+// Pieces staged through registers are written at lane position
+// 16 q + (r + 2 (q + 4 c)) % 16 for (row r, quarter q, chunk c): the 8 lanes that
+// hold one row's 8 pieces write 8 different 16-byte bank groups, and a read is
+// still one permuted 1 KiB run.
+//
+// Bound: HBM for narrow layers (524,288 x 128 -> 128: 112 us, 4.8 TB/s, a copy's
+// rate); for wide ones the fragment reads (12 KiB per 32 MFMAs and wave at
+// 256 x 256) and the MFMAs, which contend.  Measured: 65,536 x 1024 -> 1024 fp16
+// 1055 -> 200 us between other calls, 236 in a loop of its own, 65,536 x 512 -> 512 fp32 642 -> 303 us (113
+// TFLOP/s) against restaging the weight per 64 rows and 256 columns; without the
+// loads 198 us, with every fragment read from one address 219 us.
+__device__ __attribute__((aligned(16))) uint32_t g_lg_zero16[4] = {0u, 0u, 0u, 0u};
+typedef __fp16 lg_half4 __attribute__((ext_vector_type(4)));
+
+struct LinearGemmArgs {
+  const float* x;
+  const void* w;
+  const float* bias;
+  float* y;
+  int64_t rows, row_tiles;
+  int in, out, col_tiles;
+  int wkind, relu;
+};
+
+// 16 bytes per lane from src to LDS byte address lds_wave + 16 lane (below 64 KiB).
+__device__ __forceinline__ void lg_dma16(const void* src, uint32_t lds_wave) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds_wave))
+      : "memory");
+}
+
+template <int NW, int WM, int WN>
+struct LgLds {
+  static constexpr int kX = 2 * WM * 2 * 1024, kW = NW / 2 * WN * 2 * 1024;  // bytes per buffer
+  static constexpr int kBytes = 2 * (kX + kW);
+};
+
+template <bool F16, bool TILED, int NW, int WM, int WN>
+__global__ __launch_bounds__(64 * NW, 2) void linear_gemm_kernel(LinearGemmArgs a) {
+  using LD = LgLds<NW, WM, WN>;
+  constexpr int NN = NW / 2;           // waves across the outputs (two across the rows)
+  constexpr int BM = 32 * WM, BN = 16 * NN * WN;
+  constexpr int NX = WM * 4 / NW;      // row pieces per thread and step (WN weight pieces)
+  constexpr int PR = 8 * NW;           // rows between a thread's pieces
+  constexpr int KS = F16 ? 64 : 32;    // columns per step, two chunks
+  constexpr int PK = KS / 8;           // columns per 16-byte fragment piece
+  static_assert(!TILED || 2 * LD::kW <= 64 * 1024, "DMA targets below 64 KiB");
+  extern __shared__ f32x4 lo_smem[];
+  uint8_t* const sw = reinterpret_cast<uint8_t*>(lo_smem);  // W buffers first
+  uint8_t* const sx = sw + 2 * LD::kW;
+  const int tid = int(threadIdx.x), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / NN, wn = wave % NN;
+  const int r = lane & 15, q = lane >> 4;
+  // Blocks of one XCD (consecutive multiples of 8) take the column tiles of a
+  // row tile one after the other, so its x rows are read from HBM once.
+  const int64_t b = blockIdx.x;
+  const int ct = int((b >> 3) % a.col_tiles);
+  const int64_t rt = ((b >> 3) / a.col_tiles) * 8 + (b & 7);
+  if (rt >= a.row_tiles) return;
+  const int64_t row0 = rt * BM;
+  const int o0 = ct * BN;
+  const int in = a.in;
+
+  // register-staged pieces: rows tid / 8 + PR i of the tile, piece tid % 8 of the step
+  const int pr = tid >> 3, pp = tid & 7;
+  const int spos = ((pp >> 2) * 64 + 16 * (pp & 3) + ((pr + 2 * pp) & 15)) * 16 + (pr >> 4) * 2048;
+  const float* const xb = a.x + row0 * in;
+  const int xlast = int(a.rows - row0 < BM ? a.rows - row0 : BM) - 1;
+  const int olast = (a.out - o0 < BN ? a.out - o0 : BN) - 1;
+  f32x4 xr[NX][F16 ? 2 : 1];
+  f32x4 wr[TILED ? 1 : WN][F16 ? 2 : 1];
+
+  auto load = [&](int k0, int buf) {
+    const bool ok = k0 + pp * PK < in;  // a piece past `in` re-reads the step's first one and is zeroed when parked
+    const int kk = k0 + (ok ? pp * PK : 0);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) h[i] = wt[base + ((k & 15) + i) * 16];
+    for (int i = 0; i < NX; ++i) {
+      const int rr = min(pr + PR * i, xlast);
+#pragma unroll
+      for (int v = 0; v < (F16 ? 2 : 1); ++v) xr[i][v] = reinterpret_cast<const f32x4*>(xb + int64_t(rr) * in + kk)[v];
+    }
+    if constexpr (TILED) {
+      // BN outputs x 4 k tiles of 512 bytes; a wave's instruction moves two neighbouring k tiles
+#pragma unroll
+      for (int i = 0; i < WN; ++i) {
+        const int u = NW * i + wave;            // 1 KiB unit: output tile u / 2, k tiles 2 (u % 2), + 1
+        const int ot = min(u >> 1, olast >> 4);
+        const int kt = (k0 >> 4) + 2 * (u & 1) + (lane >> 5);
+        const int piece = (lane & 31) ^ ((lane & 16) >> 1);  // rows 12..15 of a tile before rows 8..11
+        const half_t* src = static_cast<const half_t*>(a.w) + (int64_t((o0 >> 4) + ot) * (in >> 4) + kt) * 256 + 8 * piece;
+        lg_dma16(16 * kt < in ? static_cast<const void*>(src) : g_lg_zero16,
+                 uint32_t(reinterpret_cast<uintptr_t>(sw + buf * LD::kW + u * 1024)));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < WN; ++i) {
+        const int o = o0 + min(pr + PR * i, olast);
+        const int64_t e = int64_t(o) * in + kk;
+        if (F16 && a.wkind == RDV_WKIND_F16_TILED16) {  // a tile copy that is not 16-byte aligned
+          const half_t* wt = static_cast<const half_t*>(a.w) + (int64_t(o >> 4) * (in >> 4) + (kk >> 4)) * 256 + (o & 15);
+          half8 h;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) h[j] = wt[((kk & 15) + j) * 16];
+          wr[i][0] = __builtin_bit_cast(f32x4, h);
+        } else if (F16 && a.wkind == RDV_WKIND_F16) {
+          wr[i][0] = *reinterpret_cast<const f32x4*>(static_cast<const half_t*>(a.w) + e);
+        } else {
+#pragma unroll
+          for (int v = 0; v < (F16 ? 2 : 1); ++v)
+            wr[i][v] = reinterpret_cast<const f32x4*>(static_cast<const float*>(a.w) + e)[v];
         }
-        v = __builtin_bit_cast(f32x4, h);
-      } else {
-        v = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.w) + int64_t(o) * a.in + k);
       }
     }
-    sw[s] = v;
-  }
-  for (int i = threadIdx.x; i < a.ob; i += kLoThreads) sb[i] = (o0 + i < a.out) ? a.bias[o0 + i] : 0.0f;
-}
-
-// Loads one wave's x for row tile `task`, columns [k0, k0 + NKC*kStep): raw[rr][c][v].
-// Rows are clamped into range (their results are never stored) and columns past
-// `in` are clamped to column 0 (zeroed on conversion), so every load is in bounds
-// and unconditional.
-template <bool F16, int RT, int NKC>
-__device__ __forceinline__ void load_x(const LinearOpArgs& a, int64_t task, int k0, int nkc, int wave, int lane,
-                                       f32x4 (&raw)[RT][NKC][LoPolicy<F16>::kVec]) {
-  using P = LoPolicy<F16>;
-  const int q = lane >> 4;
+  };
+  auto park = [&](int k0, int buf) {
+    const bool ok = k0 + pp * PK < in;
+    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int rr = 0; rr < RT; ++rr) {
-    int64_t row = (task * kLoWaves + wave) * (16 * RT) + rr * 16 + (lane & 15);
-    row = row < a.rows ? row : a.rows - 1;
-    const float* xr = a.x + row * a.in;
-#pragma unroll
-    for (int c = 0; c < NKC; ++c) {
-      if (c >= nkc) break;  // nkc is uniform: a scalar branch
-      int k = k0 + c * P::kStep + q * (P::kStep / 4);
-      k = k < a.in ? k : 0;
-#pragma unroll
-      for (int v = 0; v < P::kVec; ++v) raw[rr][c][v] = reinterpret_cast<const f32x4*>(xr + k)[v];
+    for (int i = 0; i < NX; ++i) {
+      f32x4 v;
+      if constexpr (F16) v = __builtin_bit_cast(f32x4, to_half8(xr[i][0], xr[i][1]));
+      else v = xr[i][0];
+      *reinterpret_cast<f32x4*>(sx + buf * LD::kX + spos + i * (NN * 2048)) = ok ? v : zero4;
     }
-  }
-}
-
-template <bool F16, int RT, int NKC>
-struct XFrag;
-template <int RT, int NKC>
-struct XFrag<true, RT, NKC> {
-  half8 v[RT][NKC];
-};
-template <int RT, int NKC>
-struct XFrag<false, RT, NKC> {
-  f32x4 v[RT][NKC];
-};
-
-template <bool F16, int RT, int NKC>
-__device__ __forceinline__ void convert_x(const LinearOpArgs& a, int k0, int nkc, int lane,
-                                          const f32x4 (&raw)[RT][NKC][LoPolicy<F16>::kVec],
-                                          XFrag<F16, RT, NKC>& xf) {
-  using P = LoPolicy<F16>;
-  const int q = lane >> 4;
+    if constexpr (!TILED) {
 #pragma unroll
-  for (int c = 0; c < NKC; ++c) {
-    const bool ok = c < nkc && k0 + c * P::kStep + q * (P::kStep / 4) < a.in;
-#pragma unroll
-    for (int rr = 0; rr < RT; ++rr) {
-      if constexpr (F16) {
-        const half8 h = to_half8(raw[rr][c][0], raw[rr][c][1]);
-        xf.v[rr][c] = ok ? h : half8{};
-      } else {
-        xf.v[rr][c] = ok ? raw[rr][c][0] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int i = 0; i < WN; ++i) {
+        f32x4 v = wr[i][0];
+        if constexpr (F16) {
+          if (a.wkind == RDV_WKIND_F32) v = __builtin_bit_cast(f32x4, to_half8(wr[i][0], wr[i][1]));
+        }
+        *reinterpret_cast<f32x4*>(sw + buf * LD::kW + spos + i * (NN * 2048)) = ok ? v : zero4;
       }
     }
-  }
-}
+  };
 
-template <bool F16, int RT, int NKC>
-__device__ __forceinline__ void mma_pass(const f32x4* sw, int nt, int nkc, int lane, const XFrag<F16, RT, NKC>& xf,
-                                         f32x4 (&acc)[RT][kLoMaxOb / 16]) {
+  f32x4 acc[WM][WN];
 #pragma unroll
-  for (int t = 0; t < kLoMaxOb / 16; ++t) {
-    if (t < nt) {
+  for (int n = 0; n < WN; ++n) {
+    const int col = o0 + 16 * (WN * wn + n) + 4 * q;
+    f32x4 bv;
 #pragma unroll
-      for (int c = 0; c < NKC; ++c) {
-        if (c < nkc) {
-          const f32x4 wv = sw[(t * nkc + c) * 64 + lane];
+    for (int j = 0; j < 4; ++j) bv[j] = a.bias[min(col + j, a.out - 1)];
+#pragma unroll
+    for (int m = 0; m < WM; ++m) acc[m][n] = bv;
+  }
+  load(0, 0);
+  park(0, 0);
+  if constexpr (TILED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  const int steps = (in + KS - 1) / KS;
+  for (int s = 0; s < steps; ++s) {
+    const bool more = s + 1 < steps;
+    if (more) load((s + 1) * KS, (s + 1) & 1);
+    const uint8_t* bx = sx + (s & 1) * LD::kX + wm * WM * 2048;
+    const uint8_t* bw = sw + (s & 1) * LD::kW + wn * WN * 2048;
+    // TILED, quarter q: rows 8 (q % 2) .. + 7 of k tile 2 c + q / 2, four at a time; odd
+    // quarters find theirs swapped, so neighbouring quarters read different banks
+    const uint32_t tlo = uint32_t(reinterpret_cast<uintptr_t>(bw)) + (q >> 1) * 512 + (q & 1) * 384 + r * 8;
+    const uint32_t thi = uint32_t(reinterpret_cast<uintptr_t>(bw)) + (q >> 1) * 512 + (q & 1) * 256 + 128 - (q & 1) * 128 + r * 8;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int rpos = (c * 64 + 16 * q + ((r + 2 * (q + 4 * c)) & 15)) * 16;
+      f32x4 wf[WN];
+#pragma unroll
+      for (int n = 0; n < WN; ++n) {
+        if constexpr (TILED) {
+          typedef __attribute__((address_space(3))) lg_half4 lds_h4;
+          const lg_half4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4*)(tlo + n * 2048 + c * 1024));
+          const lg_half4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4*)(thi + n * 2048 + c * 1024));
+          const f32x2 l2 = __builtin_bit_cast(f32x2, lo), h2 = __builtin_bit_cast(f32x2, hi);
+          wf[n] = f32x4{l2[0], l2[1], h2[0], h2[1]};
+        } else {
+          wf[n] = *reinterpret_cast<const f32x4*>(bw + n * 2048 + rpos);
+        }
+      }
+      f32x4 xf[WM];
+#pragma unroll
+      for (int m = 0; m < WM; ++m) xf[m] = *reinterpret_cast<const f32x4*>(bx + m * 2048 + rpos);
+      // every fragment of the chunk is on its way before its first product (2.5% over the compiler's own order)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < WM; ++m) {
+#pragma unroll
+        for (int n = 0; n < WN; ++n) {
           if constexpr (F16) {
-            const half8 wh = __builtin_bit_cast(half8, wv);
-#pragma unroll
-            for (int rr = 0; rr < RT; ++rr)
-              acc[rr][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh, xf.v[rr][c], acc[rr][t], 0, 0, 0);
+            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, wf[n]),
+                                                               __builtin_bit_cast(half8, xf[m]), acc[m][n], 0, 0, 0);
           } else {
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-              for (int rr = 0; rr < RT; ++rr)
-                acc[rr][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s], xf.v[rr][c][s], acc[rr][t], 0, 0, 0);
+            for (int k = 0; k < 4; ++k)
+              acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[n][k], xf[m][k], acc[m][n], 0, 0, 0);
           }
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    if (more) park((s + 1) * KS, (s + 1) & 1);
+    if constexpr (TILED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
   }
-}
 
-template <int RT>
-__device__ __forceinline__ void seed_bias(const float* sb, int nt, int lane, f32x4 (&acc)[RT][kLoMaxOb / 16]) {
-  const f32x4* sb4 = reinterpret_cast<const f32x4*>(sb);
 #pragma unroll
-  for (int t = 0; t < kLoMaxOb / 16; ++t) {
-    const f32x4 b = t < nt ? sb4[t * 4 + (lane >> 4)] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int rr = 0; rr < RT; ++rr) acc[rr][t] = b;
-  }
-}
-
-template <int RT>
-__device__ __forceinline__ void store_y(const LinearOpArgs& a, int64_t task, int o0, int nt, int wave, int lane,
-                                        const f32x4 (&acc)[RT][kLoMaxOb / 16]) {
-#pragma unroll
-  for (int rr = 0; rr < RT; ++rr) {
-    const int64_t row = (task * kLoWaves + wave) * (16 * RT) + rr * 16 + (lane & 15);
+  for (int m = 0; m < WM; ++m) {
+    const int64_t row = row0 + 16 * (WM * wm + m) + r;
     if (row < a.rows) {
       float* yr = a.y + row * a.out;
 #pragma unroll
-      for (int t = 0; t < kLoMaxOb / 16; ++t) {
-        const int col = o0 + 16 * t + 4 * (lane >> 4);
-        if (t < nt && col < a.out) {
-          f32x4 v = acc[rr][t];
+      for (int n = 0; n < WN; ++n) {
+        const int col = o0 + 16 * (WN * wn + n) + 4 * q;
+        if (col < a.out) {
+          f32x4 v = acc[m][n];
           if (a.relu) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = fmaxf(v[j], 0.0f);
@@ -246,59 +276,23 @@ __device__ __forceinline__ void store_y(const LinearOpArgs& a, int64_t task, int
   }
 }
 
-template <bool F16, int RT, int NKC>
-__global__ __launch_bounds__(kLoThreads) void linear_op_kernel(LinearOpArgs a) {
-  using P = LoPolicy<F16>;
-  extern __shared__ f32x4 lo_smem[];
-  const int nt = a.ob / 16;
-  const int nkc = (a.kp + P::kStep - 1) / P::kStep;
-  f32x4* sw = lo_smem;
-  float* sb = reinterpret_cast<float*>(lo_smem + nt * nkc * 64);
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // blockIdx.x = row workgroup * n_ob + output block: the blocks sharing rows
-  // are dispatched back to back, so their x re-reads hit the shared cache.
-  const int ob_idx = blockIdx.x % a.n_ob;
-  const int64_t rwg = blockIdx.x / a.n_ob;
-  const int64_t rstride = gridDim.x / a.n_ob;
-  const int o0 = ob_idx * a.ob;
-
-  f32x4 raw[RT][NKC][P::kVec];
-  XFrag<F16, RT, NKC> xf;
-  f32x4 acc[RT][kLoMaxOb / 16];
-
-  if (a.passes == 1) {
-    stage_weight<F16>(a, o0, 0, nkc, sw, sb);
-    __syncthreads();
-    int64_t task = rwg;
-    if (task >= a.tasks) return;
-    load_x<F16, RT, NKC>(a, task, 0, nkc, wave, lane, raw);
-    for (; task < a.tasks; task += rstride) {
-      convert_x<F16, RT, NKC>(a, 0, nkc, lane, raw, xf);
-      int64_t next = task + rstride;
-      next = next < a.tasks ? next : a.tasks - 1;
-      load_x<F16, RT, NKC>(a, next, 0, nkc, wave, lane, raw);
-      seed_bias<RT>(sb, nt, lane, acc);
-      mma_pass<F16, RT, NKC>(sw, nt, nkc, lane, xf, acc);
-      store_y<RT>(a, task, o0, nt, wave, lane, acc);
-    }
-    return;
+template <bool F16, bool TILED, int NW, int WM, int WN>
+int launch_linear_gemm_t(const LinearGemmArgs& a0, hipStream_t stream) {
+  constexpr int kBytes = LgLds<NW, WM, WN>::kBytes, BM = 32 * WM, BN = 8 * NW * WN;
+  LinearGemmArgs a = a0;
+  a.row_tiles = (a.rows + BM - 1) / BM;
+  a.col_tiles = (a.out + BN - 1) / BN;
+  const int64_t grid = (a.row_tiles + 7) / 8 * 8 * a.col_tiles;
+  if (grid > 0x7fffffff) return fail(RDV_ERR_UNSUPPORTED, "grid too large");
+  static bool attr = false;
+  if (!attr) {
+    RDV_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_gemm_kernel<F16, TILED, NW, WM, WN>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kBytes));
+    attr = true;
   }
-
-  // in > one pass: restage W per pass and per tile.
-  for (int64_t task = rwg; task < a.tasks; task += rstride) {
-    for (int p = 0; p < a.passes; ++p) {
-      const int k0 = p * a.kp;
-      __syncthreads();
-      stage_weight<F16>(a, o0, k0, nkc, sw, sb);
-      __syncthreads();
-      if (p == 0) seed_bias<RT>(sb, nt, lane, acc);
-      load_x<F16, RT, NKC>(a, task, k0, nkc, wave, lane, raw);
-      convert_x<F16, RT, NKC>(a, k0, nkc, lane, raw, xf);
-      mma_pass<F16, RT, NKC>(sw, nt, nkc, lane, xf, acc);
-    }
-    store_y<RT>(a, task, o0, nt, wave, lane, acc);
-  }
+  linear_gemm_kernel<F16, TILED, NW, WM, WN><<<dim3(unsigned(grid)), dim3(64 * NW), kBytes, stream>>>(a);
+  RDV_HIP_TRY(hipGetLastError());
+  return RDV_OK;
 }
 
 __global__ __launch_bounds__(256) void relu_op_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t n) {
@@ -314,17 +308,6 @@ __global__ __launch_bounds__(256) void relu_op_kernel(const float* __restrict__ 
   }
   const int64_t t = (n4 << 2) + int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (blockIdx.x == 0 && t < n) y[t] = fmaxf(x[t], 0.0f);
-}
-
-struct LoKernel {
-  const void* fn;
-  int rt;
-  int occupancy;  // resident workgroups per CU (0 = not yet queried)
-};
-
-template <bool F16, int RT, int NKC>
-const void* lo_fn() {
-  return reinterpret_cast<const void*>(&linear_op_kernel<F16, RT, NKC>);
 }
 
 }  // namespace
@@ -351,68 +334,54 @@ int linear_op_check(const rdv_linear_op_desc& d, std::string* why) {
   return RDV_OK;
 }
 
+// Tile shapes of linear_gemm_kernel and the share of the matrix rate a full chip
+// of them reaches (65,536 x 1024 -> 1024 fp16: 239, 310, 366, 418, 564 us; 65,536 x
+// 512 -> 512 fp32: 302, 333, 347, 362, 408 us).
+struct LgTile {
+  int bm, bn;
+  float eff16, eff32;
+};
+constexpr LgTile kLgTiles[] = {{256, 256, 1.0f, 1.0f}, {128, 128, 0.77f, 0.91f}, {128, 64, 0.65f, 0.87f},
+                               {64, 64, 0.57f, 0.83f}, {64, 32, 0.42f, 0.74f}};
+
+template <bool F16, bool TILED>
+int launch_linear_gemm(int tile, const LinearGemmArgs& a, hipStream_t stream) {
+  switch (tile) {
+    case 0: return launch_linear_gemm_t<F16, TILED, 8, 8, 4>(a, stream);
+    case 1: return launch_linear_gemm_t<F16, TILED, 4, 4, 4>(a, stream);
+    case 2: return launch_linear_gemm_t<F16, TILED, 4, 4, 2>(a, stream);
+    case 3: return launch_linear_gemm_t<F16, TILED, 4, 2, 2>(a, stream);
+    default: return launch_linear_gemm_t<F16, TILED, 4, 2, 1>(a, stream);
+  }
+}
+
 int launch_linear_op(const rdv_linear_op_desc& d, const float* x, const void* w, const float* bias, float* y,
                      hipStream_t stream) {
   if (d.rows == 0) return RDV_OK;
   DeviceInfo dev;
   if (int rc = device_info(&dev)) return rc;
   const bool f16 = d.precision == RDV_PREC_F16;
-  const int step = f16 ? 32 : 16;
-  const int kmax = f16 ? 256 : 128;
-  const int chunks = (d.in_features + step - 1) / step;
-  const int passes = (d.in_features + kmax - 1) / kmax;
-  const int per_pass = (chunks + passes - 1) / passes;
-  int nkc = 1;
-  while (nkc < per_pass) nkc *= 2;
-  const int rt = nkc <= 4 ? 2 : 1;
-
-  static LoKernel table[2][4] = {};  // [f16][log2 nkc]
-  int li = 0;
-  while ((1 << li) < nkc) ++li;
-  LoKernel& k = table[f16][li];
-  if (!k.fn) {
-    const void* fns[2][4] = {
-        {lo_fn<false, 2, 1>(), lo_fn<false, 2, 2>(), lo_fn<false, 2, 4>(), lo_fn<false, 1, 8>()},
-        {lo_fn<true, 2, 1>(), lo_fn<true, 2, 2>(), lo_fn<true, 2, 4>(), lo_fn<true, 1, 8>()}};
-    k.fn = fns[f16][li];
-    k.rt = rt;
+  // The tile whose busiest CU has the least work: tiles per CU, rounded up, times
+  // a tile's area over its efficiency.  Large products take the 256 x 256 tile,
+  // small ones the one that still gives every CU a block, and none pays for a
+  // last round that is nearly empty (18,624 x 512 -> 512 fp32: 122 us with 128 x
+  // 128, 584 tiles; 106 us with 128 x 64).
+  int best = 0;
+  float cost = 0.0f;
+  for (int t = 0; t < 5; ++t) {
+    const LgTile& k = kLgTiles[t];
+    const int64_t tiles = (d.rows + k.bm - 1) / k.bm * ((d.out_features + k.bn - 1) / k.bn);
+    const float c = float((tiles + dev.cu_count - 1) / dev.cu_count) * float(k.bm * k.bn) / (f16 ? k.eff16 : k.eff32);
+    if (t == 0 || c < cost) {
+      best = t;
+      cost = c;
+    }
   }
-
-  LinearOpArgs a;
-  a.x = x;
-  a.w = w;
-  a.bias = bias;
-  a.y = y;
-  a.rows = d.rows;
-  a.in = d.in_features;
-  a.out = d.out_features;
-  a.wkind = d.wkind;
-  a.relu = d.relu ? 1 : 0;
-  a.passes = passes;
-  a.kp = passes == 1 ? chunks * step : kmax;
-  a.ob = std::min(kLoMaxOb, (d.out_features + 15) / 16 * 16);
-  a.n_ob = (d.out_features + a.ob - 1) / a.ob;
-  const int64_t rows_per_task = int64_t(kLoWaves) * 16 * rt;
-  a.tasks = (d.rows + rows_per_task - 1) / rows_per_task;
-
-  const int nkc_run = (a.kp + step - 1) / step;
-  const size_t lds = size_t(a.ob / 16) * nkc_run * 64 * sizeof(f32x4) + size_t(a.ob) * sizeof(float);
-  if (lds > 64 * 1024 + kLoMaxOb * sizeof(float)) return fail(RDV_ERR_UNSUPPORTED, "linear op LDS plan too large");
-  if (!k.occupancy) {
-    RDV_HIP_TRY(hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    64 * 1024 + kLoMaxOb * int(sizeof(float))));
-  }
-  int occ = 0;
-  RDV_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k.fn, kLoThreads, lds));
-  occ = std::max(occ, 1);
-  k.occupancy = occ;
-  const int64_t slots = int64_t(dev.cu_count) * occ;
-  const int64_t rwgs = std::max<int64_t>(1, std::min<int64_t>(a.tasks, (slots + a.n_ob - 1) / a.n_ob));
-  const int64_t grid = rwgs * a.n_ob;
-  if (grid > 0x7fffffff) return fail(RDV_ERR_UNSUPPORTED, "grid too large");
-  void* params[] = {&a};
-  RDV_HIP_TRY(hipLaunchKernel(k.fn, dim3(static_cast<unsigned>(grid)), dim3(kLoThreads), params, lds, stream));
-  return RDV_OK;
+  const LinearGemmArgs a = {x, w, bias, y, d.rows, 0, d.in_features, d.out_features, 0, d.wkind, d.relu ? 1 : 0};
+  if (!f16) return launch_linear_gemm<false, false>(best, a, stream);
+  if (d.wkind == RDV_WKIND_F16_TILED16 && reinterpret_cast<uintptr_t>(w) % 16 == 0)
+    return launch_linear_gemm<true, true>(best, a, stream);
+  return launch_linear_gemm<true, false>(best, a, stream);
 }
 
 int launch_relu_op(const float* x, float* y, int64_t n, hipStream_t stream) {

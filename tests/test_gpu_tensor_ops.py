@@ -64,6 +64,36 @@ def test_linear_tensor_op_fp32_matches_oracle(shape):
     _check(op.as_type("torch").cpu().numpy(), x.numpy(), W.numpy(), b.numpy(), False, f"LinearTensorOp{shape}")
 
 
+@pytest.mark.parametrize("rows,inf,outf", [
+    (16390, 48, 1020), (4100, 80, 1000), (2050, 72, 1000), (4099, 64, 252), (70, 136, 36),  # each block tile, ragged
+    (1, 8, 4), (33, 64, 16), (257, 72, 260),   # one row; exactly one K step; one row past a tile
+])
+@pytest.mark.parametrize("kind", ["f32", "f16_w32", "f16_w16", "f16_tiled", "f16_tiled_odd"])
+def test_linear_op_tiles(rows, inf, outf, kind):
+    """Every block tile and weight kind of the linear kernel at ragged sizes, within twice the bound of any fp32
+    summation order; nothing past the last row is written.  f16_tiled_odd: a tile copy off 16-byte alignment."""
+    tiled = kind.startswith("f16_tiled")
+    if tiled:
+        inf, outf = (inf + 15) // 16 * 16, (outf + 15) // 16 * 16
+    x, W, b = _case(rows, inf, outf, seed=rows + inf)
+    f16 = kind != "f32"
+    wk, w = _lib.WKIND_F32, W.cuda()
+    if kind == "f16_w16":
+        wk, w = _lib.WKIND_F16, W.half().cuda()
+    elif tiled:
+        wk, w = _lib.WKIND_F16_TILED16, _tensor_ops.tile_weight_fp16(W.cuda())
+        if kind == "f16_tiled_odd":
+            pad = torch.empty(w.numel() + 1, dtype=torch.float16, device="cuda")
+            pad[1:] = w
+            w = pad[1:]
+    y = torch.full(((rows + 2) * outf,), 12345.0, device="cuda")
+    rc = _raw_linear(x.cuda(), w, b.cuda(), y, rows, inf, outf, _lib.PREC_F16 if f16 else _lib.PREC_F32, wk)
+    assert rc == 0, _lib.last_error()
+    out = y.cpu().numpy()
+    assert (out[rows * outf:] == 12345.0).all(), "kernel wrote past the last row"
+    _check(out[: rows * outf].reshape(rows, outf), x.numpy(), W.numpy(), b.numpy(), f16, f"{kind} {rows}x{inf}->{outf}")
+
+
 def test_relu_tensor_op_is_exact():
     x = torch.randn(64, 40)
     x[0, :8] = torch.tensor([float("nan"), float("-inf"), float("inf"), -0.0, 0.0, -1e-38, 1e-45, 3.0])
