@@ -33,6 +33,7 @@ SOURCES = [
     "volume_profile_dda.hip",
     "volume_profile_dda8.hip",
     "mlp_generic.hip",
+    "train_fused.hip",
     "train.hip",
     "winograd.hip",
     "conv_op.hip",
@@ -58,6 +59,13 @@ COMMON_FLAGS = [
 ]
 
 
+# Sources with flags of their own.  train_fused.hip: matrix products go to ordinary
+# registers unless the source asks for accumulation registers (its gradients do).
+SOURCE_FLAGS = {
+    "train_fused.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+}
+
+
 def _hipcc() -> str:
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     cand = os.path.join(rocm, "bin", "hipcc")
@@ -66,7 +74,7 @@ def _hipcc() -> str:
 
 def _compile(src: str, extra: list[str]) -> str:
     obj = os.path.join(BUILD_DIR, os.path.splitext(src)[0] + ".o")
-    cmd = [_hipcc(), *COMMON_FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [_hipcc(), *COMMON_FLAGS, *SOURCE_FLAGS.get(src, []), *extra, "-c", os.path.join(CSRC, src), "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{' '.join(cmd)}\n{res.stdout}\n{_filter(res.stderr)}")

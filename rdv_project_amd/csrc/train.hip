@@ -29,12 +29,13 @@
 //    (K = the tile's points, operands gathered from the LDS tile); dW stays in
 //    registers across the block's whole point range and is written once as a
 //    per-block partial.
-//  - train_reduce1/2_kernel: sum the per-block partials in a fixed order.
+//  - train_reduce_kernel: sums the per-block partials in a fixed order.
 #include <algorithm>
 #include <mutex>
 #include <string>
 
-#include "mlp_core.h"
+#include "train_fused.h"
+#include "train_tile.h"
 
 namespace rdv {
 
@@ -56,35 +57,6 @@ struct TrainFwdArgs {
   int64_t n;
   int has_bias;
 };
-
-// Sum over a wave (every lane gets it): DPP row shifts + row broadcasts.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float tr_dpp(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, true));
-}
-__device__ __forceinline__ float tr_wave_sum(float v) {
-  v += tr_dpp<0x111, 0xF>(v);
-  v += tr_dpp<0x112, 0xF>(v);
-  v += tr_dpp<0x114, 0xF>(v);
-  v += tr_dpp<0x118, 0xF>(v);
-  v += tr_dpp<0x142, 0xA>(v);
-  v += tr_dpp<0x143, 0xC>(v);
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-
-typedef half_t half4v __attribute__((ext_vector_type(4)));
-
-// Tile-fragment layout of the step's intermediate fp16 buffers (the kept hidden
-// activations h_i, the head gradient g and the gradients g_i between backward
-// launches), [rows][W] with rows a multiple of 64: 32-point tiles of
-// Wp = 16 ceil(W / 16) features, tile k at k 32 Wp; within a tile, 16-byte chunk
-// c = 64 s + 32 hh + col holds point col, features 16 s + 4 hh + 0..3 and then
-// 16 s + 8 + 4 hh + 0..3 (tfl_feature).  That chunk is lane 32 hh + col's B
-// fragment of K chunk s in the hidden (chunk_sigma) order, and equally the fp16
-// of D registers 8 (s % 2) .. + 7 of 32-row block s / 2, so a wave writes or
-// reads a whole 1 KiB slot s with one 16-byte access per lane.  Features past W
-// are stored as zeros.
-__device__ __forceinline__ int tfl_feature(int s, int hh, int j) { return 16 * s + 4 * hh + (j & 3) + ((j >> 2) << 3); }
 
 __global__ __launch_bounds__(kTrFwdThreads, 1) void train_fwd_kernel(TrainFwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -992,52 +964,52 @@ __global__ __launch_bounds__(kTpThreads, 1) void train_pair_kernel(TrainPairArgs
   }
 }
 
-// All of a step's reductions in two launches, in a fixed order (so dW is the
-// same run to run).  Job j sums its partials part_j[b][i] over b < nb_j into
-// out_j[i] = scale * sum, i < count_j; the jobs' elements are concatenated
-// (job j at start[j]) and so are their blocks (job j's first block bstart[j],
-// 256 elements per block), so a block's job is wave-uniform.
-//  stage 1: mid[s][e] = sum of part[b][i] for b = s, s + S, s + 2S, ... (in order)
-//  stage 2: out[i] = scale * sum over s < S of mid[s][e] (in order)
-constexpr int kTrSplit = 32;
+// All of a step's reductions in one launch, in a fixed order (so dW is the same
+// run to run).  Job j sums its partials part_j[b][i] over b < nb_j into
+// out_j[i] = scale * sum, i < count_j; the jobs' blocks are concatenated (job
+// j's first block bstart[j], kTrRedElems elements per block), so a block's job is
+// wave-uniform.  A block's threads are kTrRedElems elements x kTrRedSplit runs of
+// partials (run s takes b = s, s + S, ...; eight loads in flight), and the runs
+// are added in order through LDS.  Bound: reading the partials; a first launch
+// over 32 runs and a second over their sums took 12.5 us for the 15.7 MB of
+// 32 -> 64 x 4 -> 16, most of it the two launches' latency.
+constexpr int kTrRedElems = 32, kTrRedSplit = 8;
 constexpr int kTrMaxJobs = 2 * RDV_MLP_MAX_LAYERS + 1;
 struct ReduceJobs {
   int n;
   const float* part[kTrMaxJobs];
   float* out[kTrMaxJobs];
   int nb[kTrMaxJobs];
-  int64_t start[kTrMaxJobs + 1];
+  int count[kTrMaxJobs];
   int bstart[kTrMaxJobs + 1];
 };
 
-__device__ __forceinline__ int reduce_job(const ReduceJobs& J) {
+__global__ __launch_bounds__(kTrRedElems * kTrRedSplit) void train_reduce_kernel(ReduceJobs J, float scale) {
+  __shared__ float sums[kTrRedSplit][kTrRedElems];
   int j = 0;
   while (j + 1 < J.n && int(blockIdx.x) >= J.bstart[j + 1]) ++j;
-  return j;
-}
-
-__global__ void train_reduce1_kernel(ReduceJobs J, float* __restrict__ mid) {
-  const int j = reduce_job(J);
-  const int64_t count = J.start[j + 1] - J.start[j];
-  const int64_t i = int64_t(int(blockIdx.x) - J.bstart[j]) * 256 + threadIdx.x;
-  if (i >= count) return;
-  const int s = blockIdx.y;
-  const float* part = J.part[j];
+  const int count = J.count[j], nb = J.nb[j];
+  const int e = int(threadIdx.x) % kTrRedElems, s = int(threadIdx.x) / kTrRedElems;
+  const int i = (int(blockIdx.x) - J.bstart[j]) * kTrRedElems + e;
+  const float* part = J.part[j] + (i < count ? i : 0);
   float acc = 0.0f;
-  for (int b = s; b < J.nb[j]; b += kTrSplit) acc += part[int64_t(b) * count + i];
-  mid[int64_t(s) * J.start[J.n] + J.start[j] + i] = acc;
-}
-
-__global__ void train_reduce2_kernel(ReduceJobs J, const float* __restrict__ mid, float scale) {
-  const int j = reduce_job(J);
-  const int64_t count = J.start[j + 1] - J.start[j];
-  const int64_t i = int64_t(int(blockIdx.x) - J.bstart[j]) * 256 + threadIdx.x;
-  if (i >= count) return;
-  const int64_t total = J.start[J.n];
-  float acc = 0.0f;
-#pragma unroll 8
-  for (int s = 0; s < kTrSplit; ++s) acc += mid[int64_t(s) * total + J.start[j] + i];
-  J.out[j][i] = acc * scale;
+  int b = s;
+  for (; b + 7 * kTrRedSplit < nb; b += 8 * kTrRedSplit) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = part[int64_t(b + k * kTrRedSplit) * count];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc += v[k];
+  }
+  for (; b < nb; b += kTrRedSplit) acc += part[int64_t(b) * count];
+  sums[s][e] = acc;
+  __syncthreads();
+  if (s == 0 && i < count) {
+    float t = acc;
+#pragma unroll
+    for (int k = 1; k < kTrRedSplit; ++k) t += sums[k][e];
+    J.out[j][i] = t * scale;
+  }
 }
 
 // Every transposed-weight pack of a step in one launch.  Job k writes the
@@ -1110,34 +1082,6 @@ struct TrainPair2Args {
 };
 
 constexpr int kT2Threads = 512;  // 8 waves: two roles of 4
-
-// 0/1 fragment par: lane (n = lane % 32, hh = lane / 32), element j is 1 where
-// tfl_feature(par, hh, j) == n.  A x select(0) + A' x select(1) turns the K
-// slots of two consecutive 16-feature chunks (or of the two 16-point halves of
-// a K = points fragment pair) into the 32 columns of D.
-__device__ __forceinline__ half8 tp2_select(int par, int lane) {
-  half8 v;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = tfl_feature(par, lane >> 5, j) == (lane & 31) ? half_t(1.0f) : half_t(0.0f);
-  return v;
-}
-
-// D registers 8 ks .. 8 ks + 7 as fp16 (points tfl_feature(ks, h, 0..7) of a
-// point-major product; features 32 block + tfl_feature(ks, h, 0..7) of a
-// feature-major one).
-__device__ __forceinline__ half8 tp2_half(const f32x16& d, int ks) {
-  half8 v;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = half_t(d[8 * ks + j]);
-  return v;
-}
-
-// Sum of 8 fp16 values into an fp32 accumulator.
-__device__ __forceinline__ float tp2_sum(const half8& v, float acc) {
-#pragma unroll
-  for (int j = 0; j < 8; j += 2) acc = __builtin_amdgcn_fdot2(half2v{v[j], v[j + 1]}, half2v{1, 1}, acc, false);
-  return acc;
-}
 
 // LDS carve-up of train_pair2_kernel (half8 units): three input buffers
 // (g_l slots, then h_{l-1} slots) and two exchange buffers (g_l and h_{l-1} as
@@ -1377,15 +1321,6 @@ __global__ __launch_bounds__(kT2Threads, 1) void train_pair2_kernel(TrainPair2Ar
 // tiles, each reading the tile's x (2 KiB) from L2.
 constexpr int kB0Threads = 256;
 
-// 0/1 fragment for the natural feature order of chunk par: lane (n, hh),
-// element j is 1 where 16 par + 8 hh + j == n.
-__device__ __forceinline__ half8 tp2_select_nat(int par, int lane) {
-  half8 v;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = 16 * par + 8 * (lane >> 5) + j == (lane & 31) ? half_t(1.0f) : half_t(0.0f);
-  return v;
-}
-
 __global__ __launch_bounds__(kB0Threads, 2) void train_bwd0_kernel(TrainBwdArgs a) {
   const int tid = int(threadIdx.x);
   const int lane = tid & 63;
@@ -1453,7 +1388,7 @@ struct TrainPlan {
   int blocks_fwd, blocks_bwd, blocks_pair;
   bool keep[RDV_MLP_MAX_LAYERS];   // h_i stored by the forward
   int64_t wt_off[RDV_MLP_MAX_LAYERS], h_off[RDV_MLP_MAX_LAYERS], g_off, dz_off[2], dw_off[RDV_MLP_MAX_LAYERS],
-      db_off[RDV_MLP_MAX_LAYERS], loss_off, mid_off;
+      db_off[RDV_MLP_MAX_LAYERS], loss_off;
   int64_t total;
 };
 
@@ -1580,7 +1515,7 @@ static void train_plan(const rdv_mlp_desc& d, const MlpLayout& lay, int64_t n, i
     all += int64_t(d.dims[i + 1]) * (d.dims[i] + 1);
   }
   p->loss_off = take(int64_t(p->blocks_fwd) * 4);
-  p->mid_off = take(int64_t(kTrSplit) * all * 4);
+  take(int64_t(32) * all * 4);  // unused: keeps the workspace size, and with it what the static scratch accepts
   p->total = off;
 }
 
@@ -1602,6 +1537,44 @@ int launch_train_step(const rdv_mlp_desc& d, const MlpLayout& lay, const void* p
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   const int L = d.n_layers;
   const uint8_t* pk = static_cast<const uint8_t*>(packed);
+  const float scale = 1.0f / float(double(n) * d.dims[L]);
+  ReduceJobs jobs;
+  jobs.n = 0;
+  jobs.bstart[0] = 0;
+  // queues the reduction of part[nb][count] into out (run after the backward)
+  auto reduce = [&](const float* part, int nb, int64_t count, float* out) -> int {
+    const int j = jobs.n++;
+    jobs.part[j] = part;
+    jobs.out[j] = out;
+    jobs.nb[j] = nb;
+    jobs.count[j] = int(count);
+    jobs.bstart[j + 1] = jobs.bstart[j] + int((count + kTrRedElems - 1) / kTrRedElems);
+    return RDV_OK;
+  };
+  auto reduce_all = [&]() -> int {
+    train_reduce_kernel<<<dim3(unsigned(jobs.bstart[jobs.n])), dim3(kTrRedElems * kTrRedSplit), 0, stream>>>(jobs, scale);
+    RDV_HIP_TRY(hipGetLastError());
+    return RDV_OK;
+  };
+  if (train_fused_ok(d)) {
+    // one kernel for the whole step; its loss partials take the place of the
+    // gradients between backward launches, which it does not have
+    const int nb = train_fused_blocks(d, n, di.cu_count);
+    float* parts_w[RDV_MLP_MAX_LAYERS];
+    float* parts_b[RDV_MLP_MAX_LAYERS];
+    for (int l = 0; l < L; ++l) {
+      parts_w[l] = reinterpret_cast<float*>(ws + p.dw_off[l]);
+      parts_b[l] = reinterpret_cast<float*>(ws + p.db_off[l]);
+    }
+    float* lp = reinterpret_cast<float*>(ws + p.dz_off[0]);
+    rc = launch_train_fused(d, lay, packed, x, target, n, nb, lp, parts_w, parts_b, stream);
+    if (rc == RDV_OK) rc = reduce(lp, nb, 1, loss);
+    for (int l = 0; l < L && rc == RDV_OK; ++l) {
+      rc = reduce(parts_w[l], nb, int64_t(d.dims[l + 1]) * d.dims[l], dW[l]);
+      if (rc == RDV_OK) rc = reduce(parts_b[l], nb, d.dims[l + 1], db[l]);
+    }
+    return rc == RDV_OK ? reduce_all() : rc;
+  }
   // forward groups
   static bool attr_set = false;
   if (!attr_set) {
@@ -1647,21 +1620,6 @@ int launch_train_step(const rdv_mlp_desc& d, const MlpLayout& lay, const void* p
     }
     RDV_HIP_TRY(hipGetLastError());
   }
-  const float scale = 1.0f / float(double(n) * d.dims[L]);
-  ReduceJobs jobs;
-  jobs.n = 0;
-  jobs.start[0] = 0;
-  jobs.bstart[0] = 0;
-  // queues the reduction of part[nb][count] into out (run after the backward)
-  auto reduce = [&](const float* part, int nb, int64_t count, float* out) -> int {
-    const int j = jobs.n++;
-    jobs.part[j] = part;
-    jobs.out[j] = out;
-    jobs.nb[j] = nb;
-    jobs.start[j + 1] = jobs.start[j] + count;
-    jobs.bstart[j + 1] = jobs.bstart[j] + int((count + 255) / 256);
-    return RDV_OK;
-  };
   rc = reduce(reinterpret_cast<float*>(ws + p.loss_off), p.blocks_fwd, 1, loss);
   if (rc != RDV_OK) return rc;
   // backward: layer pairs from the head down, then layer 0 alone if L is odd;
@@ -1795,13 +1753,7 @@ int launch_train_step(const rdv_mlp_desc& d, const MlpLayout& lay, const void* p
     rc = reduce(ba.db_part, p.blocks_bwd, out, db[0]);
     if (rc != RDV_OK) return rc;
   }
-  float* mid = reinterpret_cast<float*>(ws + p.mid_off);
-  const unsigned gx = unsigned(jobs.bstart[jobs.n]);
-  train_reduce1_kernel<<<dim3(gx, kTrSplit), dim3(256), 0, stream>>>(jobs, mid);
-  RDV_HIP_TRY(hipGetLastError());
-  train_reduce2_kernel<<<dim3(gx), dim3(256), 0, stream>>>(jobs, mid, scale);
-  RDV_HIP_TRY(hipGetLastError());
-  return RDV_OK;
+  return reduce_all();
 }
 
 }  // namespace rdv

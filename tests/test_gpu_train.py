@@ -175,3 +175,24 @@ def test_c5_full_config_against_cpu_restatement():
         torch.set_num_threads(threads)
     _check(loss, [(torch.from_numpy(dw), torch.from_numpy(db)) for dw, db in grads], ref_loss, ref,
            "C5 full size vs the CPU restatement")
+
+
+@pytest.mark.parametrize("n", [1, 33, 1000, 20011])  # one point; a tile and a point; ragged; several tiles per wave
+@pytest.mark.parametrize("dims", [
+    [16, 32, 8], [48] + [32] * 5 + [16], [64] + [32] * 4 + [8],               # 32 wide, 1 to 5 hidden layers
+    [16, 64, 16], [32] + [64] * 4 + [16], [48, 64, 64, 8], [64] + [64] * 4 + [8],  # 64 wide, 1 to 4; 1 to 4 input chunks
+])
+def test_narrow_chains(dims, n):
+    """The chains one kernel trains (equal hidden widths of 32 or 64), at the edges of its tiles and input chunks,
+    against the oracle at the step's bars: loss 1e-4, per layer 1e-2 of the gradient's norm."""
+    g = torch.Generator().manual_seed(len(dims) * 100 + n)
+    layers = []
+    for i in range(len(dims) - 1):
+        lim = (6.0 / dims[i]) ** 0.5
+        layers.append((((torch.rand(dims[i + 1], dims[i], generator=g) * 2 - 1) * lim).half().float(),
+                       torch.randn(dims[i + 1], generator=g) * 0.1))
+    x = torch.randn(n, dims[0], generator=g).half()
+    t = torch.randn(n, dims[-1], generator=g)
+    loss, grads = rdv.mse_backward(_chain(layers), x.cuda(), t.cuda())
+    ref_loss, ref_grads = T.mse_grads(x.float().numpy(), [(w.numpy(), b.numpy()) for w, b in layers], t.numpy())
+    _check(loss.item(), grads, ref_loss, ref_grads, f"{dims} n={n}")
