@@ -21,14 +21,15 @@
 //   from global memory for every (position, channel block) pair, .h:113-137) is
 //   replaced by one staging of the haloed input in LDS per tile group.
 //
-// Work decomposition (generic kernel, any layout and dtype): a tile group is 16
+// Work decomposition (strip kernel: channels-last with cin off a multiple of 4, or
+// x not aligned for the patch kernel's vectors): a tile group is 16
 // consecutive tiles of one tile row (2 output rows x 32 output columns).  Each
 // block owns a contiguous range of groups; per group it stages the 4 x 34 x CIN
 // input region in LDS (fp32), transforms it to V in B-fragment order (fp16),
 // then every wave evaluates its 16 output channels for the 16 tiles.  NCHW fp16
-// input takes winograd3x3_pipe_kernel (below): the same transforms and GEMMs,
-// input rows by DMA, and the input transform of one tile row overlapped with
-// the GEMMs of the previous one.
+// input with W % 8 == 0 takes winograd3x3_pipe_kernel (below): the same transforms
+// and GEMMs, input rows by DMA, and the input transform of one tile row overlapped
+// with the GEMMs of the previous one; every other input winograd3x3_patch_kernel.
 #include <algorithm>
 #include <type_traits>
 
@@ -379,6 +380,171 @@ __global__ __launch_bounds__(256, 2) void winograd3x3_kernel(WinogradArgs a) {
   }
 }
 
+
+// --------------------------------------------------------- patch kernel
+// winograd3x3_patch_kernel: any layout whose patches load as vectors: channels-last
+// (cin a multiple of 4, 16-byte loads of 4 channels; 8-byte for fp16), and NCHW
+// (dwords; fp16 rows of an even width are whole dwords).  A thread owns one tile
+// and four channels of a 16-tile group and loads its 4 x 4 patch straight into
+// registers (the overlap of neighbouring patches is served by the L1), a group
+// ahead, so the loads are in flight during the current group's GEMMs; V goes
+// to one of two LDS buffers as B fragments, so a group costs one barrier.  Its V,
+// GEMMs and inverse transform are winograd3x3_kernel's, operation for operation.
+//
+// Bound: issue.  Per group and wave ~130 adds, 32 conversions and 16 LDS writes
+// for V, 32 MFMAs with a fragment read each, the inverse transform; U's 32 KiB per
+// wave and the first patches are the fixed part.  Against staging the region in
+// LDS with 4-byte loads and index arithmetic per element (same bits): 256 x 256,
+// 48 -> 48, channels-last fp32 33.1 -> 16.5 us, fp16 33.3 -> 12.2; 130 x 254, 64 ->
+// 128, NCHW fp16 40.8 -> 25.0 (48 dword loads per thread and group), fp32 40.4 -> 34.0.
+enum { kPatchHwcF32 = 0, kPatchHwcF16 = 1, kPatchChwF16 = 2, kPatchChwF32 = 3 };
+
+template <int MODE>
+struct WgPatch {
+  // raw registers: [row][column] vectors of 4 channels, or [row][dword of a row][channel]
+  using vec = typename std::conditional<MODE == kPatchHwcF32, f32x4,
+                                        typename std::conditional<MODE == kPatchHwcF16, half4, uint32_t>::type>::type;
+  static constexpr int kCols = MODE == kPatchChwF16 ? 3 : 4;
+  static constexpr int kCh = MODE == kPatchHwcF32 || MODE == kPatchHwcF16 ? 1 : 4;
+  vec v[4][kCols][kCh];
+};
+
+template <int KC, int MODE>
+__global__ __launch_bounds__(256, 2) void winograd3x3_patch_kernel(WinogradArgs a) {
+  using P = WgPatch<MODE>;
+  constexpr bool HWC = MODE == kPatchHwcF32 || MODE == kPatchHwcF16;
+  constexpr bool F16 = MODE == kPatchHwcF16 || MODE == kPatchChwF16;
+  using in_t = typename std::conditional<F16, half_t, float>::type;
+  __shared__ half8 sv[2][16 * KC * 64];                  // V fragments [p][kc][lane]
+  const int tid = int(threadIdx.x), lane = tid & 63;
+  const int g = blockIdx.y * 4 + (tid >> 6);             // output channel group (16 channels)
+  const bool active = 16 * g < a.cout;
+  const int hw = a.H * a.W, tw = a.W / 2;
+  // this thread's tile of a group and first channel; HWC: consecutive threads walk
+  // a pixel's channels, CHW: neighbouring tiles
+  const int n = HWC ? tid / (8 * KC) : tid & 15;
+  const int ci0 = 4 * (HWC ? tid % (8 * KC) : tid >> 4);
+  const bool loader = n < 16 && ci0 < 32 * KC;
+  const bool real = loader && ci0 < a.cin;
+  const int cl = ci0 < a.cin ? ci0 : 0;
+  const in_t* const xc = static_cast<const in_t*>(a.x) + (HWC ? cl : cl * hw);
+  // channels past cin (CHW's last quartet): loaded from the quartet's first
+  int chs[P::kCh];
+#pragma unroll
+  for (int c = 0; c < P::kCh; ++c) chs[c] = cl + c < a.cin ? c * hw : 0;
+
+  const int64_t per_block = (a.ngroups + gridDim.x - 1) / gridDim.x;
+  const int64_t g_begin = int64_t(blockIdx.x) * per_block;
+  const int64_t g_end = g_begin + per_block < a.ngroups ? g_begin + per_block : a.ngroups;
+
+  // Every load is in bounds (rows and columns clamped) and unconditional; the
+  // zero border is applied when the patch is used.
+  auto load = [&](int64_t grp, P& p) {
+    const int seg = int(grp % a.seg);
+    const int64_t rest = grp / a.seg;
+    const int tr = int(rest % a.th);
+    const int img = int(rest / a.th);
+    const in_t* base = xc + int64_t(img) * a.cin * hw;
+    const int tc = min(seg * kWgTiles + n, tw - 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int ih = min(max(2 * tr - 1 + r, 0), a.H - 1);
+#pragma unroll
+      for (int c = 0; c < P::kCols; ++c) {
+        if constexpr (HWC) {
+          const int iw = min(max(2 * tc - 1 + c, 0), a.W - 1);
+          p.v[r][c][0] = *reinterpret_cast<const typename P::vec*>(base + (ih * a.W + iw) * a.cin);
+        } else {
+          // fp16: columns 2 tc - 2 + 2 c and the next; fp32: column 2 tc - 1 + c
+          const int iw = F16 ? min(max(2 * tc - 2 + 2 * c, 0), a.W - 2) : min(max(2 * tc - 1 + c, 0), a.W - 1);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            p.v[r][c][k] = *reinterpret_cast<const uint32_t*>(base + chs[k] + ih * a.W + iw);
+        }
+      }
+    }
+  };
+  // patch element (row r, column c) of the four channels, in fp32
+  auto at = [&](const P& p, int r, int c) {
+    f32x4 d;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (MODE == kPatchHwcF32) {
+        d[k] = p.v[r][c][0][k];
+      } else if constexpr (MODE == kPatchHwcF16) {
+        const half4 hv = p.v[r][c][0];
+        d[k] = float(hv[k]);
+      } else if constexpr (MODE == kPatchChwF16) {
+        const half2v hv = __builtin_bit_cast(half2v, p.v[r][(c + 1) / 2][k]);
+        d[k] = float(hv[(c + 1) & 1]);
+      } else {
+        const uint32_t w = p.v[r][c][k];
+        d[k] = __builtin_bit_cast(float, w);
+      }
+    }
+    return d;
+  };
+
+  P cur;
+  if (loader && g_begin < g_end) load(g_begin, cur);
+  // this wave's U fragments, resident for the whole block (their loads follow the first patches')
+  half8 u[16][KC];
+  const int g_n = (a.cout + 15) / 16;
+  const int gu = active ? g : 0;
+#pragma unroll
+  for (int p = 0; p < 16; ++p)
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc)
+      u[p][kc] = reinterpret_cast<const half8*>(a.U)[((int64_t(p) * KC + kc) * g_n + gu) * 64 + lane];
+  const f32x4 bias = wg_lane_bias(a, gu, lane);
+
+  for (int64_t grp = g_begin; grp < g_end; ++grp) {
+    const int seg = int(grp % a.seg);
+    const int64_t rest = grp / a.seg;
+    const int tr = int(rest % a.th);
+    const int img = int(rest / a.th);
+    half8* const svb = sv[(grp - g_begin) & 1];
+    if (loader) {
+      const int tc = min(seg * kWgTiles + n, tw - 1);
+      // zero border: row 0 of the first tile row, row 3 of the last, and the same for columns
+      f32x4 d[4][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool rok = real && (r == 0 ? tr > 0 : r == 3 ? tr + 1 < a.th : true);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const bool ok = rok && (c == 0 ? tc > 0 : c == 3 ? tc + 1 < tw : true);
+          d[r][c] = at(cur, r, c);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) d[r][c][k] = ok && (HWC || ci0 + k < a.cin) ? d[r][c][k] : 0.0f;
+        }
+      }
+      const int kc = ci0 / 32, k = ci0 % 32;
+      const int flane = (k / 8) * 16 + n, j0 = k % 8;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // row r of m = B^T d, then of V = m B, in _winograd_fwd's order
+        f32x4 m[4], vv[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          m[c] = r == 0 ? d[0][c] - d[2][c] : r == 1 ? d[1][c] + d[2][c] : r == 2 ? d[2][c] - d[1][c] : d[1][c] - d[3][c];
+        vv[0] = m[0] - m[2];
+        vv[1] = m[1] + m[2];
+        vv[2] = m[2] - m[1];
+        vv[3] = m[1] - m[3];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          half4 hv = {half_t(vv[b][0]), half_t(vv[b][1]), half_t(vv[b][2]), half_t(vv[b][3])};
+          half_t* dst = reinterpret_cast<half_t*>(&svb[((4 * r + b) * KC + kc) * 64 + flane]) + j0;
+          *reinterpret_cast<half4*>(dst) = hv;
+        }
+      }
+    }
+    if (loader && grp + 1 < g_end) load(grp + 1, cur);  // in flight during this group's GEMMs
+    __syncthreads();  // V complete; the other buffer's readers are a group behind
+    if (active) wg_gemm_store<KC>(u, svb, lane, g, bias, a, img, tr, seg);
+  }
+}
 
 // ------------------------------------------------------- NCHW fp16 fast path
 // For NCHW fp16 input with W % 8 == 0 (the benchmark layout).  Input rows arrive
@@ -897,21 +1063,32 @@ int launch_winograd3x3(const rdv_conv_desc& d, const void* x, const void* U, con
   int64_t blocks = (2 * int64_t(di.cu_count) + slices - 1) / slices;  // ~2 resident blocks per CU
   if (a.ngroups < blocks) blocks = a.ngroups;
   const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(slices)), block(256);
+  // Patches of whole vectors: channels-last quartets, NCHW dwords.  The strip kernel stays for the rest (element loads).
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x);
+  if (chw ? xa % 4 == 0 : d.cin % 4 == 0 && xa % (f16 ? 8 : 16) == 0) {
+#define RDV_WG_PATCH(MODE) \
+  if (d.cin <= 32) winograd3x3_patch_kernel<1, MODE><<<grid, block, 0, stream>>>(a); else winograd3x3_patch_kernel<2, MODE><<<grid, block, 0, stream>>>(a)
+    if (chw && f16) { RDV_WG_PATCH(kPatchChwF16); }
+    else if (chw) { RDV_WG_PATCH(kPatchChwF32); }
+    else if (f16) { RDV_WG_PATCH(kPatchHwcF16); }
+    else { RDV_WG_PATCH(kPatchHwcF32); }
+#undef RDV_WG_PATCH
+    RDV_HIP_TRY(hipGetLastError());
+    return RDV_OK;
+  }
   if (d.cin <= 32) {
     if (f16) {
       if (chw) winograd3x3_kernel<1, true, true><<<grid, block, 0, stream>>>(a);
       else winograd3x3_kernel<1, true, false><<<grid, block, 0, stream>>>(a);
     } else {
-      if (chw) winograd3x3_kernel<1, false, true><<<grid, block, 0, stream>>>(a);
-      else winograd3x3_kernel<1, false, false><<<grid, block, 0, stream>>>(a);
+      winograd3x3_kernel<1, false, false><<<grid, block, 0, stream>>>(a);
     }
   } else {
     if (f16) {
       if (chw) winograd3x3_kernel<2, true, true><<<grid, block, 0, stream>>>(a);
       else winograd3x3_kernel<2, true, false><<<grid, block, 0, stream>>>(a);
     } else {
-      if (chw) winograd3x3_kernel<2, false, true><<<grid, block, 0, stream>>>(a);
-      else winograd3x3_kernel<2, false, false><<<grid, block, 0, stream>>>(a);
+      winograd3x3_kernel<2, false, false><<<grid, block, 0, stream>>>(a);
     }
   }
   RDV_HIP_TRY(hipGetLastError());

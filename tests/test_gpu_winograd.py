@@ -241,3 +241,28 @@ def test_c3_unaligned_out_view(c3_oracle):
     y = conv(x.cuda(), relu=True, out=view)
     torch.cuda.synchronize()
     _check_close(y.float().cpu().numpy()[0].transpose(1, 2, 0), c3_oracle, "C3 unaligned out vs oracle", f16_out=True)
+
+
+@pytest.mark.parametrize("H,W", [(2, 2), (6, 30), (4, 34), (10, 66)])  # one tile; a short, an exact + 1 and a third group
+@pytest.mark.parametrize("cin,cout", [(4, 16), (20, 32), (36, 80), (64, 48)])  # one and two K chunks, partial ones
+@pytest.mark.parametrize("layout,dtype", [(_lib.LAYOUT_HWC, _lib.DTYPE_F32), (_lib.LAYOUT_HWC, _lib.DTYPE_F16),
+                                          (_lib.LAYOUT_CHW, _lib.DTYPE_F16), (_lib.LAYOUT_CHW, _lib.DTYPE_F32)])
+def test_patch_kernel_edges(H, W, cin, cout, layout, dtype):
+    """Patches loaded as vectors, every layout and type, at the edges of images, tile groups and channel chunks."""
+    rng = np.random.default_rng(H * W + cin)
+    x = rng.uniform(-1, 1, (2, H, W, cin)).astype(np.float16).astype(np.float32)
+    w = rng.normal(0, 0.2, (3, 3, cin, cout)).astype(np.float32)
+    b = rng.normal(0, 0.5, cout).astype(np.float32)
+    y = _run(x, w, b, layout, dtype, layout, _lib.DTYPE_F32, False, batch=2)
+    for i in range(2):
+        _check_close(y[i], O.winograd_conv(x[i], w, b), f"image {i}")
+
+
+@pytest.mark.parametrize("cin,dtype", [(13, _lib.DTYPE_F32), (6, _lib.DTYPE_F16)])
+def test_strip_kernel_odd_channels(cin, dtype):
+    """Channels-last with cin off a multiple of 4 keeps the element-wise kernel."""
+    rng = np.random.default_rng(cin)
+    x = rng.uniform(-1, 1, (1, 6, 36, cin)).astype(np.float16).astype(np.float32)
+    w = rng.normal(0, 0.2, (3, 3, cin, 16)).astype(np.float32)
+    y = _run(x, w, None, _lib.LAYOUT_HWC, dtype, _lib.LAYOUT_HWC, _lib.DTYPE_F32, False)
+    _check_close(y[0], O.winograd_conv(x[0], w, np.zeros(16, np.float32)), f"cin {cin}")
