@@ -104,6 +104,26 @@ __device__ __forceinline__ void gen_sources(const uint8_t* packed, const GenNet&
   }
 }
 
+// GenFieldNet's head value at up to 32 points, of lanes 0 .. 31 (half of
+// gen_field_pair64's work).
+__device__ __forceinline__ float gen_field_single32(const half8* w0, const float* b0, bool has_bias, int lane, int h,
+                                                    const float (&p)[3], int act) {
+  using N = GenFieldNet;
+  const int z = opaque_zero();
+  const LdsWeights ws{w0 + z, lane};
+  half8 b[N::kMaxKC];
+  f32x16 acc0[N::kMaxMT], acc1[N::kMaxMT];
+  build_input<N>(p, h, b);
+  if (has_bias) {
+    load_bias<N, 0>(acc0, b0 + z, h);
+    run_chain<N, 0, true, true>(ws, b, acc0, acc1, b0 + z, h);
+  } else {
+    run_chain<N, 0, true, false>(ws, b, acc0, acc1, b0, h);
+  }
+  // the last layer's result is in set (kL - 1) % 2
+  return gen_head_act(act, 0, (N::kL - 1) % 2 == 0 ? acc0[0][0] : acc1[0][0]);
+}
+
 // The chain's head value of row 0 at this lane's sample p (3 coordinates).
 // F32L: the chain may hold exact fp32 layers (gen_chain_mixed).
 template <int MT, bool F32L = false>
@@ -115,21 +135,8 @@ __device__ __forceinline__ float gen_field_row0(const GenNet& g, const half8* w0
   auto get = [&](int d) { return d == 0 ? p[0] : (d == 1 ? p[1] : p[2]); };
   float v = 0.0f;
   if constexpr (!F32L && MT >= 2) {
-    if (g.fast) {  // GenFieldNet (gen_net checked the shape and layout): the compiled chain
-      using N = GenFieldNet;
-      const LdsWeights ws{wsrc, lane};
-      half8 b[N::kMaxKC];
-      f32x16 acc0[N::kMaxMT], acc1[N::kMaxMT];
-      build_input<N>(p, h, b);
-      if (has_bias) {
-        load_bias<N, 0>(acc0, b0 + z, h);
-        run_chain<N, 0, true, true>(ws, b, acc0, acc1, b0 + z, h);
-      } else {
-        run_chain<N, 0, true, false>(ws, b, acc0, acc1, b0, h);
-      }
-      // the last layer's result is in set (kL - 1) % 2
-      return gen_head_act(act, 0, (N::kL - 1) % 2 == 0 ? acc0[0][0] : acc1[0][0]);
-    }
+    // GenFieldNet (gen_net checked the shape and layout): the compiled chain
+    if (g.fast) return gen_field_single32(w0, b0, has_bias, lane, h, p, act);
   }
   auto sink = [&](const auto& acc) { v = gen_head_act(act, 0, acc[0][0]); };
   if constexpr (F32L) {
@@ -164,30 +171,49 @@ __device__ __forceinline__ float gen_field_pair64(const half8* w0, const float* 
   return gen_head_act(act, 0, h == 0 ? accA[0][0] : vb);
 }
 
+// voxel_majorant_field.h: the cell of axis coordinate x in a grid of dim cells.
+__device__ __forceinline__ int voxel_cell(float x, int dim) {
+#pragma clang fp contract(off)
+  const float fd = float(dim);
+  // int() truncates toward zero; clamping first keeps the conversion in range
+  // (and sends NaN to 0) without changing any in-range result.
+  const float f = (x * 0.5f + 0.5f) * fd;
+  return int(fminf(fmaxf(f, 0.0f), fd - 1.0f));
+}
+
+// The index of the voxel holding x (voxel_majorant's).
+__device__ __forceinline__ int64_t voxel_index(int mw, int mh, int md, const float (&x)[3]) {
+  return (int64_t(voxel_cell(x[2], md)) * mh + voxel_cell(x[1], mh)) * mw + voxel_cell(x[0], mw);
+}
+
+// The voxel holding x, and per axis the distance along w to its later face.
+__device__ __forceinline__ int64_t voxel_exits(int mw, int mh, int md, const float (&x)[3], const float (&w)[3],
+                                               float (&te)[3]) {
+#pragma clang fp contract(off)
+  const int dim[3] = {mw, mh, md};
+  int cell[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    cell[i] = voxel_cell(x[i], dim[i]);
+    const float vs = 2.0f / float(dim[i]);
+    const float bmin = float(cell[i]) * vs - 1.0f;
+    const float bmax = bmin + vs;
+    // the later of the two face distances: rounded division is monotonic, so the
+    // sign of w names it (one division per axis); w = 0 or NaN takes both
+    te[i] = ((w[i] > 0.0f ? bmax : bmin) - x[i]) / w[i];
+    if (!(fabsf(w[i]) > 0.0f)) te[i] = fmaxf(te[i], (bmax - x[i]) / w[i]);
+  }
+  return (int64_t(cell[2]) * mh + cell[1]) * mw + cell[0];
+}
+
 // voxel_majorant_field.h: the majorant of the voxel holding x and the distance
 // along w to that voxel's exit.
 __device__ __forceinline__ float voxel_majorant(const float* __restrict__ grid, int mw, int mh, int md,
                                                 const float (&x)[3], const float (&w)[3], float& dist) {
-#pragma clang fp contract(off)
-  const int dim[3] = {mw, mh, md};
-  int cell[3];
   float te[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const float fd = float(dim[i]);
-    // int() truncates toward zero; clamping first keeps the conversion in range
-    // (and sends NaN to 0) without changing any in-range result.
-    const float f = (x[i] * 0.5f + 0.5f) * fd;
-    cell[i] = int(fminf(fmaxf(f, 0.0f), fd - 1.0f));
-    const float vs = 2.0f / fd;
-    const float bmin = float(cell[i]) * vs - 1.0f;
-    const float bmax = bmin + vs;
-    const float t0 = (bmin - x[i]) / w[i];
-    const float t1 = (bmax - x[i]) / w[i];
-    te[i] = fmaxf(t0, t1);
-  }
+  const int64_t v = voxel_exits(mw, mh, md, x, w, te);
   dist = fminf(fminf(te[0], te[1]), te[2]);
-  return grid[(int64_t(cell[2]) * mh + cell[1]) * mw + cell[0]];
+  return grid[v];
 }
 
 // Raises `kernel`'s dynamic-LDS limit to kGenFieldLdsCap, once per kernel.

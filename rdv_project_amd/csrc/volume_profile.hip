@@ -36,10 +36,21 @@ namespace rdv {
 // environment rays are VolumeProfile's.
 //
 // Mapping: as the ratio-tracking kernel, a wave holds 32 rays (lanes l and l + 32 mirror ray
-// l); each lane runs its ray's state machine until it needs an extinction value, then the
-// wave evaluates the extinction chain once for the 32 pending points.  The environment and
-// albedo maps are evaluated afterwards over the recorded directions and positions
-// (rdv_volume_profile_finish combines them).
+// l), or 64 where the chain is the compiled GenFieldNet; each lane runs its ray's state
+// machine until it needs an extinction value, then the wave evaluates the extinction chain
+// once for the pending points.  The environment and albedo maps are evaluated afterwards over
+// the recorded directions and positions (rdv_volume_profile_finish combines them).
+//
+// Bound by the rounds of the waves that hold the longest rays: a round is one evaluation of
+// the chain plus whatever the slowest lane has to do between two points.  Three things keep
+// that short (512 x 512 rays, 16 environment samples, 5-layer 64-wide chain: 10.25 ms without
+// them, 6.99 with; 180 x 100 rays, 4 samples: 4.88 and 2.30):
+//   - a step inside a march runs by itself (vp_march_step); the state machine's other parts
+//     run when half of the wave's rays wait for them;
+//   - a tracked ray that grazes a voxel face takes its flights without divisions or logarithms;
+//   - a launch's rays are spread over every CU, and a wave with at most 32 rays evaluates one
+//     tile a round.
+// None changes what a ray computes or draws, so outputs are the same bits for every schedule.
 struct VpArgs {
   const float* rays;
   int64_t nrays;
@@ -381,11 +392,16 @@ __device__ __forceinline__ void vp_start(const VpCtx& c, VpRay& r, int64_t ray) 
   else vp_depth_begin<DDA>(c, r, ray);
 }
 
-// Advances ray `ray` until it needs the extinction at a point (true, the point
-// in q) or has finished (false).  has / sigma: the extinction at the point the
-// previous call asked for.
+// What vp_advance leaves a ray as: finished, waiting for the extinction at q, or
+// to be called again (a long run of grazing flights, taken kVpGrazeRun at a time
+// so that the wave's other rays are not held up).
+enum : int { kVpFinished = 0, kVpPoint = 1, kVpYield = 2 };
+constexpr int kVpGrazeRun = 32;
+
+// Advances ray `ray` until it needs the extinction at a point (in q) or has
+// finished.  has / sigma: the extinction at the point the previous call asked for.
 template <bool DDA>
-__device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray, bool has, float sigma,
+__device__ __forceinline__ int vp_advance(const VpCtx& c, VpRay& r, int64_t ray, bool has, float sigma,
                                            float (&q)[3]) {
 #pragma clang fp contract(off)
   const VpArgs& a = c.a;
@@ -402,7 +418,7 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
           }
         }
         vp_point(r.x, r.wo, r.t, q);
-        return true;
+        return kVpPoint;
       case kVpDepth:
         if (has) {
           has = false;
@@ -426,7 +442,7 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
           }
         }
         vp_point(r.x, r.wo, r.t, q);
-        return true;
+        return kVpPoint;
       case kVpTauDda:  // volume_profile_dda.h:53-77
         if constexpr (DDA) {
           if (has) {
@@ -438,11 +454,11 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
               break;
             }
           }
-          if (vp_dda_walk(c, r, q)) return true;
+          if (vp_dda_walk(c, r, q)) return kVpPoint;
           vp_depth_begin<DDA>(c, r, ray);
           break;
         } else {
-          return false;
+          return kVpFinished;
         }
       case kVpDepthDda:  // volume_profile_dda.h:83-129
         if constexpr (DDA) {
@@ -467,11 +483,11 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
               break;
             }
           }
-          if (vp_dda_walk(c, r, q)) return true;
+          if (vp_dda_walk(c, r, q)) return kVpPoint;
           vp_after_depth(c, r, ray);
           break;
         } else {
-          return false;
+          return kVpFinished;
         }
       case kVpRm:  // raymarching_transmittance_trait.h
         if (has) {
@@ -496,7 +512,7 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) q[i] = r.p[i];
-        return true;
+        return kVpPoint;
       case kVpRt: {  // ratiotracking_transmittance_trait.h
         bool end = false;
         if (has) {
@@ -511,25 +527,53 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
             }
           }
         }
+        // A ray almost parallel to a voxel face it has come to takes flights of the
+        // least length (1e-6) that do not move its coordinate across that face in
+        // fp32, up to the 1024-step cap (some hundred paths of a 512 x 512 frame,
+        // whose waves waited for 1024 whole flights: 30% of the frame's time).
+        // While an axis stands still within 1e-6 of its face the next distance is
+        // 1e-6 without a division, and the majorant changes only with the voxel.
+        float te[3], mj = 0.0f;
+        int64_t vox = -1;
+        bool graze = false, stuck[3] = {false, false, false};
+        int run = 0;
         while (!end) {
+          if (graze && ++run > kVpGrazeRun) return kVpYield;
           if (!(r.d > 0.0f && r.k < 1024)) break;
-          float dist;
-          float mj = voxel_majorant(a.majorant, a.mw, a.mh, a.md, r.p, r.dl, dist);
-          mj = fmaxf(mj, 1e-12f);
-          dist = fmaxf(dist, 1e-6f);
+          float dist = 1e-6f;
+          if (!graze) {
+            vox = voxel_exits(a.mw, a.mh, a.md, r.p, r.dl, te);
+            mj = fmaxf(a.majorant[vox], 1e-12f);
+            dist = fmaxf(fminf(fminf(te[0], te[1]), te[2]), 1e-6f);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) stuck[i] = te[i] <= 1e-6f;
+          } else {
+            const int64_t v = voxel_index(a.mw, a.mh, a.md, r.p);
+            if (v != vox) mj = fmaxf(a.majorant[v], 1e-12f);
+            vox = v;
+          }
           const float u = rng_uniform(r.st);
-          const float ff = -logf(1.0f - u) / (mj * c.nee_ds);
-          const float dt = fminf(dist, ff);
+          const float m = mj * c.nee_ds;
+          // -log(1 - u) >= u (u has 23 bits, so 1 - u is exact): with u past dist m, and
+          // a margin for the logarithm's rounding, the voxel's exit cuts the flight
+          // whatever its exact length
+          float dt = dist;
+          if (!(m > 0.0f && u > dist * m * 1.001f)) dt = fminf(dist, -logf(1.0f - u) / m);
           r.d = r.d - dt;
 #pragma unroll
-          for (int i = 0; i < 3; ++i) r.p[i] = r.p[i] + dt * r.dl[i];
+          for (int i = 0; i < 3; ++i) {
+            const float pn = r.p[i] + dt * r.dl[i];
+            stuck[i] = stuck[i] && pn == r.p[i];
+            r.p[i] = pn;
+          }
+          graze = stuck[0] || stuck[1] || stuck[2];
           ++r.k;
           if (dt >= dist) continue;
           if (r.d <= 0.0f) break;
           r.maj = mj;
 #pragma unroll
           for (int i = 0; i < 3; ++i) q[i] = r.p[i];
-          return true;
+          return kVpPoint;
         }
         a.env_w[ray * a.es + r.s] = r.S * r.T;
         ++r.s;
@@ -537,9 +581,44 @@ __device__ __forceinline__ bool vp_advance(const VpCtx& c, VpRay& r, int64_t ray
         break;
       }
       default:
-        return false;
+        return kVpFinished;
     }
   }
+}
+
+// One step of a march that stays in its phase: applies the extinction sigma and
+// forms the next point (true).  A step that ends the march, crosses a threshold
+// or leaves a DDA cell is left untouched for vp_advance (false).
+template <bool DDA>
+__device__ __forceinline__ bool vp_march_step(const VpCtx& c, VpRay& r, float sigma, float (&q)[3]) {
+#pragma clang fp contract(off)
+  const VpArgs& a = c.a;
+  if (r.phase == kVpRm) {
+    const float T = r.T + (sigma * c.nee_ds) * a.step;
+    const float d = r.d - a.step;
+    if (T > 16.0f || !(d > 0.0f && r.k + 1 < 4096)) return false;
+    r.T = T;
+    r.d = d;
+    ++r.k;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      r.p[i] = r.p[i] + a.step * c.ldo[i];
+      q[i] = r.p[i];
+    }
+    return true;
+  }
+  const bool first = r.phase == (DDA ? kVpTauDda : kVpTau);
+  if (!first && r.phase != (DDA ? kVpDepthDda : kVpDepth)) return false;
+  const float tau = (first ? r.tau : r.ctau) + (sigma * a.density_scale) * a.step;
+  const float t = r.t + a.step;
+  if (tau > 20.0f || !(t < (DDA ? r.d : r.tmax)) || r.k + 1 >= kVpMaxMarch) return false;
+  if (!first && tau * r.scale >= r.tcross) return false;
+  if (first) r.tau = tau;
+  else r.ctau = tau;
+  r.t = t;
+  ++r.k;
+  vp_point(r.x, r.wo, t, q);
+  return true;
 }
 
 struct VpGenArgs {
@@ -547,6 +626,12 @@ struct VpGenArgs {
   const uint8_t* packed;
   GenNet net;
 };
+
+// A wave's waiting rays are served when they are at least 1 / kVpWaitShare of its
+// rays (or none marches).  512 x 512 rays, 16 environment samples each, 5-layer
+// 64-wide extinction chain: share 2 7.0 ms, 3 7.3, 4 7.3, 6 7.2; 180 x 100 rays
+// within 1% of one another.
+constexpr int kVpWaitShare = 2;
 
 // One block's rays (DDA: VolumeProfileDDA's marches, a compile-time choice so that
 // VolumeProfile's kernel carries none of the walk's state).  W64: 64 rays per
@@ -588,14 +673,33 @@ __device__ __forceinline__ void volume_profile_body(const VpGenArgs& ga) {
   bool exhausted = false;  // the block's range has run dry
   float q[3] = {0.0f, 0.0f, 0.0f};
   float sigma = 0.0f;
+  // A block with at most 32 rays for each of its waves gives every wave its share
+  // at once and evaluates one tile a round: the time is then the longest ray's
+  // rounds, and a wave that took 64 rays would leave others without any.
+  const int waves = int(blockDim.x) >> 6;
+  const int share = (nr + waves - 1) / waves;
+  const bool narrow = share <= 32;
+  if (narrow && (W64 ? lane : col) >= share) exhausted = true;
   const uint64_t below = (uint64_t(1) << (W64 ? lane : col)) - 1;
   const bool owner = W64 || h == 0;  // the lane whose ballot bit stands for its ray
   for (;;) {
-    for (;;) {
+    // Marches step here; everything else (a march's end, a threshold, a DDA cell's
+    // exit, a tracked ray's flights, the next ray) waits until a share of the
+    // wave's rays does: that code is ten times a step's length, and with 64 rays
+    // some ray needed it in nearly every round, the others standing by.  What a
+    // ray computes does not depend on when it runs.
+    if (ray >= 0 && has && vp_march_step<DDA>(c, r, sigma, q)) {
+      pending = true;
+      has = false;
+    }
+    const int waiting = __builtin_popcountll(__builtin_amdgcn_ballot_w64(owner && !pending && (ray >= 0 || !exhausted)));
+    const int marching = __builtin_popcountll(__builtin_amdgcn_ballot_w64(owner && pending));
+    while (waiting * kVpWaitShare >= waiting + marching) {  // all of the wave's rays that wait, then no more
       if (ray >= 0 && !pending) {
-        pending = vp_advance<DDA>(c, r, ray, has, sigma, q);
+        const int state = vp_advance<DDA>(c, r, ray, has, sigma, q);
         has = false;
-        if (!pending) ray = -1;
+        pending = state == kVpPoint;
+        if (state == kVpFinished) ray = -1;
       }
       const bool idle = ray < 0 && !exhausted;
       const uint64_t want = __builtin_amdgcn_ballot_w64(owner && idle);
@@ -618,13 +722,17 @@ __device__ __forceinline__ void volume_profile_body(const VpGenArgs& ga) {
         }
       }
     }
-    if (__builtin_amdgcn_ballot_w64(owner && pending) == 0) break;  // every ray is out of work
+    if (__builtin_amdgcn_ballot_w64(owner && pending) == 0) {
+      if (__builtin_amdgcn_ballot_w64(owner && ray >= 0) == 0) break;  // every ray is out of work
+      continue;  // only grazing rays left
+    }
     float p[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) p[i] = pending ? q[i] : 0.0f;
     float s;
     if constexpr (W64) {
-      s = gen_field_pair64(w0, b0, has_bias, lane, h, p, act);
+      if (narrow) s = gen_field_single32(w0, b0, has_bias, lane, h, p, act);
+      else s = gen_field_pair64(w0, b0, has_bias, lane, h, p, act);
     } else {
       s = gen_field_row0<MT, F32L>(g, w0, b0, has_bias, lane, h, p, act);
       s = __shfl(s, col);  // the value of lane col (row 0 of its column)
@@ -653,10 +761,16 @@ __global__ __launch_bounds__(64 * gen_waves<2>(), 1) void volume_profile64_kerne
   volume_profile_body<2, true, DDA, false, true>(ga);
 }
 
+// Work items of a launch (launch_gen_field takes one per wave): 8 rays each, so
+// that a small launch spreads over every CU; a ray's steps run one after the other
+// whatever shares its wave (18,000 rays on the 36 CUs that 64 per wave fill: 3.3 ms,
+// the length of the longest rays at two waves per SIMD).
+static int64_t vp_items(int64_t nrays) { return (nrays + 7) / 8; }
+
 // Launch of volume_profile64_kernel<DDA> (64 rays per wave).
 template <bool DDA>
 static int launch_volume_profile64(const VpGenArgs& ga, int64_t nrays, int cu, hipStream_t stream) {
-  return launch_gen_field<VpGenArgs, 2, true>(&volume_profile64_kernel<DDA>, ga, (nrays + 63) / 64, cu,
+  return launch_gen_field<VpGenArgs, 2, true>(&volume_profile64_kernel<DDA>, ga, vp_items(nrays), cu,
                                                gen_lds_bytes(ga.net), stream);
 }
 
@@ -749,9 +863,9 @@ int launch_volume_profile(const rdv_mlp_desc& d, const MlpLayout& lay, const voi
     return dda_grid != nullptr ? launch_volume_profile64<true>(ga, nrays, di.cu_count, stream)
                                : launch_volume_profile64<false>(ga, nrays, di.cu_count, stream);
   // 32 rays per wave
-  if (dda_grid != nullptr) return launch_volume_profile_dda_any(ga, (nrays + 31) / 32, di.cu_count, mixed, stream);
-  if (mixed) RDV_GEN_FIELD_DISPATCH_MIXED(volume_profile_kernel, ga, (nrays + 31) / 32, di.cu_count, ga.net, stream);
-  RDV_GEN_FIELD_DISPATCH(volume_profile_kernel, ga, (nrays + 31) / 32, di.cu_count, ga.net, stream,
+  if (dda_grid != nullptr) return launch_volume_profile_dda_any(ga, vp_items(nrays), di.cu_count, mixed, stream);
+  if (mixed) RDV_GEN_FIELD_DISPATCH_MIXED(volume_profile_kernel, ga, vp_items(nrays), di.cu_count, ga.net, stream);
+  RDV_GEN_FIELD_DISPATCH(volume_profile_kernel, ga, vp_items(nrays), di.cu_count, ga.net, stream,
                          launch_volume_profile8);
 }
 

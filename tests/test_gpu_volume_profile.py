@@ -348,6 +348,63 @@ def test_sensor_dda_non_cubic_grid_and_transform():
     _check(img.reshape(-1, vp.OUT), ws, ref, 22 * 16, len(thr), 2, 2, 1e-5, 1e-6, 1.0, True, "DDA sensor")
 
 
+@pytest.mark.parametrize("dims,dda", [([3, 64, 64, 64, 1], False), ([3, 64, 64, 64, 1], True), ([3, 32, 32, 1], False),
+                                      ([3, 160, 1], True)])
+def test_rays_do_not_depend_on_the_launch(dims, dda):
+    """A ray's outputs are the same bits whichever rays share its wave: the first
+    n of a launch that fills every wave against launches of n rays (one, a
+    remainder past one tile, the sizes at which a block's waves hold 32 rays
+    and one more)."""
+    layers = _rand_field(dims, seed=sum(dims))
+    ext = _field(layers, head="softplus")
+    maj = torch.from_numpy(_majorant_of(_np(layers), "softplus", 3)[..., None]).cuda()
+    head = [ext, rdv.TensorGrid(maj)]
+    if dda:
+        head.append(rdv.TensorGrid((maj > maj.median()).float()))
+    kind = rdv.VolumeProfileDDA if dda else rdv.VolumeProfile
+    vp = kind(*head, rdv.Constant([1.0, 0.8]), rdv.Constant([0.3, 0.5]), [0.8, 0.4], density_scale=2.0, g=0.2,
+              step_size=0.05, environment_samples=2)
+    rays = _camera_rays(320, 260)
+    full = _run(vp, rays, (5, 6, 7, 8))[0]
+    for n in (1, 33, 65, 1000, 65536, 65537):
+        np.testing.assert_array_equal(_run(vp, rays[:n].copy(), (5, 6, 7, 8))[0], full[:n], err_msg=f"{n} rays")
+
+
+@pytest.mark.parametrize("res", [4, (3, 5, 4)])
+def test_grazing_rays_match_oracle(res):
+    """Environment rays that start on a voxel face (x = 0.5 of a grid with 4
+    columns) almost parallel to it: flights of the least length that leave x
+    where it is, up to the step cap.  Their weights against the oracle's at the
+    bar that holds for all (an ulp of a logarithm may move a draw)."""
+    res = (res,) * 3 if isinstance(res, int) else res
+    sigma, sd, es = 0.9, 2, 3
+    rng = np.random.default_rng(9)
+    maj = rng.uniform(0.9, 1.8, res).astype(np.float32)
+    n = 3000
+    rays = np.zeros((n, 6), np.float32)
+    rays[:, 0] = 0.5
+    rays[:, 1] = rng.uniform(-0.95, 0.95, n)
+    rays[:, 2] = -1.5
+    rays[:, 3] = 1e-30  # x stays at 0.5 along the ray
+    rays[:, 5] = 1.0
+    ext = _field(_const_layers(sigma))
+    vp = rdv.VolumeProfile(ext, rdv.TensorGrid(torch.from_numpy(maj[..., None]).cuda()), rdv.Constant([1.0, 0.5]),
+                           rdv.Constant([0.4, 0.6]), [0.9, 0.6], density_scale=1.3, step_size=0.02,
+                           environment_samples=es)
+    seeds = (3, 1, 4, 1)
+    out, ws, n = _run(vp, rays, seeds)
+    ref = V.volume_profile(rays, lambda p: np.full(p.shape[0], sigma, np.float32), maj, seeds, [0.9, 0.6], sd,
+                           environment_samples=es, step_size=0.02, density_scale=1.3,
+                           albedo=lambda p: np.tile(np.float32([0.4, 0.6]), (p.shape[0], 1)),
+                           environment=lambda w: np.tile(np.float32([1.0, 0.5]), (w.shape[0], 1)))
+    _check(out, ws, ref, n, 2, sd, es, 1e-5, 1e-6, 1.0, True, "grazing rays")
+    wx = ref["dirs"][:, 0, 0]
+    grazing = (ref["valid"] == 1) & (wx < 0) & (wx > -0.025)  # 1e-6 |wx| below half an ulp of 0.5
+    assert grazing.sum() >= 10
+    w0 = ws["wts"][: n * es].reshape(n, es)[grazing, 0]
+    assert np.isclose(w0, ref["wts"][grazing, 0], rtol=1e-5, atol=1e-6).mean() >= 0.98
+
+
 def test_full_size_properties():
     """512 x 512 C4 camera rays through a constant medium: S is the closed form
     1 - exp(-sigma ds L) to the march's step, and the mean ratio-tracked
