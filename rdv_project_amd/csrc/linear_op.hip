@@ -50,11 +50,11 @@ __device__ __forceinline__ half8 to_half8(f32x4 a, f32x4 b) {
 // still one permuted 1 KiB run.
 //
 // Bound: HBM for narrow layers (524,288 x 128 -> 128: 112 us, 4.8 TB/s, a copy's
-// rate); for wide ones the fragment reads (12 KiB per 32 MFMAs and wave at
-// 256 x 256) and the MFMAs, which contend.  Measured: 65,536 x 1024 -> 1024 fp16
-// 1055 -> 200 us between other calls, 236 in a loop of its own, 65,536 x 512 -> 512 fp32 642 -> 303 us (113
-// TFLOP/s) against restaging the weight per 64 rows and 256 columns; without the
-// loads 198 us, with every fragment read from one address 219 us.
+// rate); for wide ones the tiles' stores: a chip's tiles run in step, so every CU
+// writes its 256 KiB at once and computes nothing meanwhile (65,536 x 1024 -> 1024
+// fp16: 141 us of 199 without the stores).  Measured against restaging the weight
+// per 64 rows and 256 columns: that shape 1055 -> 199 us, 65,536 x 512 -> 512 fp32
+// 642 -> 280 us (123 TFLOP/s).
 __device__ __attribute__((aligned(16))) uint32_t g_lg_zero16[4] = {0u, 0u, 0u, 0u};
 typedef __fp16 lg_half4 __attribute__((ext_vector_type(4)));
 
