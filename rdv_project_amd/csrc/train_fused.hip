@@ -59,6 +59,11 @@ struct FusedNet {
   // dW accumulators (32 x 32 blocks): layer 0 [MT][MTI], hidden [MT][MT] each, head [1][MT]
   static constexpr int dw(int l) { return l == 0 ? 0 : MT * MTI + (l - 1) * MT * MT; }
   static constexpr int kAcc = dw(D) + MT;
+  // Blocks held in accumulation registers, of which a wave has 256 (fused_dw): the
+  // first 16.  Any after those (the head's, at 64 wide, 4 deep and past 32 inputs) are
+  // ordinary registers.
+  static constexpr int kAgpr = kAcc < 16 ? kAcc : 16;
+  static_assert(kAgpr * 16 <= 256 && kAcc - kAgpr <= 2, "dW in registers");
   // stages of a tile, each with its weight fragments: forward layers 0 .. D (the
   // head), then the transposed ones of layers D .. 1
   static constexpr int kStages = 2 * D + 1;
@@ -95,8 +100,11 @@ __device__ __forceinline__ half8 fused_mask(const half8& g, const half8& h) {
 // acc += a0 b0 + a1 b1 with acc in accumulation registers.  Written out so that
 // only the dW blocks live there: the compiler's own choice, made for a whole
 // function, puts the short-lived products there too and then moves every value
-// back before its conversion (560 moves per tile).  Nothing but these chains
-// touches acc until the end of the tile loop (fused_dw_done).
+// back before its conversion (560 moves per tile).  The compiler does not know
+// these for products and puts no wait before an access of acc: nothing else may
+// touch it inside the tile loop, so the blocks must fit the file (kAgpr; a 17th
+// makes the compiler move blocks in and out between products), and
+// fused_dw_done ends every tile.
 __device__ __forceinline__ void fused_dw(f32x16& acc, const half8& a0, const half8& b0, const half8& a1, const half8& b1) {
   asm volatile(
       "s_nop 1\n\t"
@@ -105,8 +113,14 @@ __device__ __forceinline__ void fused_dw(f32x16& acc, const half8& a0, const hal
       : "+a"(acc)
       : "v"(a0), "v"(b0), "v"(a1), "v"(b1));
 }
-// The wait a read of acc needs after its last product.
-__device__ __forceinline__ void fused_dw_done() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+// The wait a read of acc needs after its last product, at the end of each tile
+// (32 of its ~10,000 cycles); every later read depends on it.
+template <int N>
+__device__ __forceinline__ void fused_dw_done(f32x16 (&acc)[N]) {
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
+}
 
 template <int MT, int D, int MTI>
 __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(TrainFusedArgs a) {
@@ -200,9 +214,11 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
   const half8 nat0 = tp2_select_nat(0, lane), nat1 = tp2_select_nat(1, lane);
   __syncthreads();
 
-  f32x16 acc[N::kAcc];
+  f32x16 acc[N::kAgpr], accv[N::kAcc > N::kAgpr ? N::kAcc - N::kAgpr : 1];
 #pragma unroll
-  for (int i = 0; i < N::kAcc; ++i) acc[i] = f32x16{};
+  for (int i = 0; i < N::kAgpr; ++i) acc[i] = f32x16{};
+#pragma unroll
+  for (int i = N::kAgpr; i < N::kAcc; ++i) accv[i - N::kAgpr] = f32x16{};
   float db[D * MT + 1];
 #pragma unroll
   for (int i = 0; i <= D * MT; ++i) db[i] = 0.0f;
@@ -312,7 +328,13 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
 #pragma unroll
         for (int t = 0; t < (l == 0 ? MTI : MT); ++t) {
           const int k = N::dw(l) + o * (l == 0 ? MTI : MT) + t;
-          fused_dw(acc[k], g0, ht[t][0], g1, ht[t][1]);
+          if (k < N::kAgpr) {
+            fused_dw(acc[k < N::kAgpr ? k : 0], g0, ht[t][0], g1, ht[t][1]);
+          } else {
+            f32x16& v = accv[k < N::kAgpr ? 0 : k - N::kAgpr];
+            v = __builtin_amdgcn_mfma_f32_32x32x16_f16(g0, ht[t][0], v, 0, 0, 0);
+            v = __builtin_amdgcn_mfma_f32_32x32x16_f16(g1, ht[t][1], v, 0, 0, 0);
+          }
         }
       }
       if (l > 0) {
@@ -331,9 +353,9 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
         }
       }
     }
+    fused_dw_done(acc);
   }
 
-  fused_dw_done();
   // ---- the block's sums: loss, db, then dW in rounds of RB blocks (every wave
   // writes its RB blocks to LDS, wave w sums block w over the waves in order)
   constexpr int RB = N::kRB;
@@ -353,7 +375,8 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
       if (k0 + k < N::kAcc) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const f32x16& v = acc[k0 + k < N::kAcc ? k0 + k : 0];
+          const int b = k0 + k;
+          const f32x16& v = b < N::kAgpr ? acc[b < N::kAgpr ? b : 0] : accv[b < N::kAcc && b >= N::kAgpr ? b - N::kAgpr : 0];
           red[((k * NW + wave) * 4 + q) * 64 + lane] = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
         }
       }
@@ -420,7 +443,7 @@ static const FusedKernel* fused_kernel(int mt, int depth, int mti) {
 }
 
 // The chain's kernel, or nullptr: equal hidden widths of 32 (up to 5 layers) or
-// 64 (up to 4: a fifth's dW no longer fits the registers), at most 64 inputs and
+// 64 (up to 4: a fifth's dW fits no registers, FusedNet::kAgpr), at most 64 inputs and
 // 16 outputs.
 static const FusedKernel* fused_for(const rdv_mlp_desc& d) {
   const int L = d.n_layers, hw = d.dims[1];

@@ -196,3 +196,25 @@ def test_narrow_chains(dims, n):
     loss, grads = rdv.mse_backward(_chain(layers), x.cuda(), t.cuda())
     ref_loss, ref_grads = T.mse_grads(x.float().numpy(), [(w.numpy(), b.numpy()) for w, b in layers], t.numpy())
     _check(loss.item(), grads, ref_loss, ref_grads, f"{dims} n={n}")
+
+
+@pytest.mark.parametrize("inputs", [32, 48, 64])
+def test_narrow_head_rows(inputs):
+    """Every row of the head's gradient, 16 outputs behind four 64-wide layers (at 48 and 64 inputs the head's blocks
+    do not fit the accumulation registers), at several tiles per wave: a row that lost a sixteenth of its points would
+    be 25% off.  1e-2 of each row's norm, the step's bar."""
+    dims, n = [inputs] + [64] * 4 + [16], 70011
+    g = torch.Generator().manual_seed(inputs)
+    layers = []
+    for i in range(len(dims) - 1):
+        lim = (6.0 / dims[i]) ** 0.5
+        layers.append((((torch.rand(dims[i + 1], dims[i], generator=g) * 2 - 1) * lim).half().float(),
+                       torch.randn(dims[i + 1], generator=g) * 0.1))
+    x = torch.randn(n, inputs, generator=g).half()
+    t = torch.randn(n, 16, generator=g)
+    loss, grads = rdv.mse_backward(_chain(layers), x.cuda(), t.cuda())
+    ref_loss, ref_grads = T.mse_grads(x.float().numpy(), [(w.numpy(), b.numpy()) for w, b in layers], t.numpy())
+    _check(loss.item(), grads, ref_loss, ref_grads, f"{dims} n={n}")
+    dw, ref = grads[-1][0].cpu().double().numpy(), ref_grads[-1][0]
+    rows = np.linalg.norm(dw - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert (rows <= 1e-2).all(), f"head rows off by {np.round(rows, 4)}"
