@@ -10,17 +10,20 @@
 //     sequence of train_fwd_kernel, so h is the same to the bit);
 //   head: g = 2 (y - t), the loss;
 //   backward, layer by layer from the head: g^T and h^T as K = points operands
-//     (each an MFMA against a 0/1 selection fragment, exact), dW += g^T h and db
-//     in registers, g_{l-1}^T = W^T g^T masked by h > 0 (W^T fragments in LDS).
+//     (through the wave's LDS scratch: point-major in, transposing reads out), dW +=
+//     g^T h and db in registers, g_{l-1}^T = W^T g^T masked by h > 0 (W^T fragments
+//     in LDS).
 // At the end a block sums its waves' dW through LDS and writes one partial.
 //
-// Bound: the matrix cores, 126 MFMAs (4,032 cycles) per tile of 32 -> 64 x 4 -> 16,
-// plus the vector ALU's hand-offs, masks and conversions, which add to them, at one
-// wave per SIMD.  262,144 points of that chain, whole step: 209 us with a kernel
-// per layer pair (run-time shapes, transposes by 2-byte LDS writes, activations
-// through memory) -> 98 us (this kernel, compiler's choice of registers) -> 62 us
-// (only dW in accumulation registers, packed masks, weights fetched a stage
-// ahead) -> 55 us (one reduction launch) -> 51 us (one round trip of staging).
+// Bound: the vector ALU's hand-offs, masks and conversions plus the matrix cores
+// (90 MFMAs, 2,880 cycles, per tile of 32 -> 64 x 4 -> 16), which add up at one wave
+// per SIMD.  262,144 points of that chain, whole step: 209 us with a kernel per
+// layer pair (run-time shapes, transposes by 2-byte LDS writes, activations through
+// memory) -> 51 us (dW in accumulation registers, packed masks, weights fetched a
+// stage ahead, one reduction launch, one round trip of staging).  Transposing by
+// products with 0/1 fragments takes 35 more MFMAs, the same time (51.0 us, here
+// 50.5; 1 to 2 layers 4 to 10% less at 2^19 points, 5 layers of 32 8% more) and
+// turns one infinity or NaN into NaN across its 32 features.
 #include <algorithm>
 
 #include "train_fused.h"
@@ -70,7 +73,10 @@ struct FusedNet {
   static constexpr int st_base(int s) { return s <= D ? fw(s) : wt(2 * D + 1 - s); }
   static constexpr int st_units(int s) { return s < D ? (s == 0 ? MT * kKC0 : MT * kKC) : s == D ? kKC : s == D + 1 ? MT : MT * kKC; }
   static constexpr int kStMax = MT * (kKC > kKC0 ? kKC : kKC0);
-  static constexpr int kLds = kUnits * 1024 + kBias * 4;
+  // a wave's transposing scratch: g_l and h_{l-1} of its tile, a row of 128 bytes per point
+  static constexpr int kTr = 32 * 128;
+  static constexpr int kTrOff = kUnits * 1024 + kBias * 4;
+  static constexpr int kLds = kTrOff + kNW * 3 * kTr;
   static constexpr int kRB = 4;                   // accumulator blocks summed per round at the end
   static constexpr int kRed = kRB * kNW * 4096;
   static constexpr int kBytes = kLds > kRed ? kLds : kRed;
@@ -120,6 +126,27 @@ __device__ __forceinline__ void fused_dw_done(f32x16 (&acc)[N]) {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
   for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
+}
+
+// A wave's transposing scratch: a row of 128 bytes per point, 32-byte slots (slot s:
+// features 16 s ..).  A row's slots are permuted by its last two bits and their
+// 16-byte halves by the third, so that the 8 lanes of a 16-byte write and the 16 of
+// a transposing read (4 rows x 32 bytes) each find different banks; slot s is at
+// the offset of slot 0 xor 32 s.
+__device__ __forceinline__ uint32_t fused_slot(int point, int s, int half) {
+  return uint32_t(point * 128 + ((s ^ (point & 3)) << 5) + ((half ^ ((point >> 2) & 1)) << 4));
+}
+
+// 8 points of a feature per lane as half a K = points operand: elements j: points
+// tfl_feature(0, hh, j) past the first row.  src: the lane's piece of its quartet of
+// rows; a transposing read hands lane i of 16 column i of the block of 4 x 16 values
+// whose 8-byte pieces the lanes point at, lane i at piece i % 4 of row i / 4.
+__device__ __forceinline__ half8 fused_points(uint32_t src) {
+  typedef __fp16 tf_half4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) tf_half4 lds_h4;
+  const half4v lo = __builtin_bit_cast(half4v, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4*)(src)));
+  const half4v hi = __builtin_bit_cast(half4v, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h4*)(src + 8 * 128)));
+  return half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
 template <int MT, int D, int MTI>
@@ -210,8 +237,11 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
 #pragma unroll
     for (int k = 0; k < BI; ++k) sb[min(k * T + tid, N::kBias - 1)] = bv[k];
   }
-  const half8 sel0 = tp2_select(0, lane), sel1 = tp2_select(1, lane);
-  const half8 nat0 = tp2_select_nat(0, lane), nat1 = tp2_select_nat(1, lane);
+  // the wave's scratch (g's part, then two of h's): this lane's point, and its piece of a transposing read
+  typedef __attribute__((address_space(3))) half8 lds_h8;
+  const uint32_t tg = uint32_t(reinterpret_cast<uintptr_t>(smem + N::kTrOff + wave * 3 * N::kTr));
+  const uint32_t put0 = fused_slot(col, 0, h);
+  const uint32_t get0 = fused_slot(4 * h + ((lane >> 2) & 3), (lane >> 4) & 1, (lane >> 1) & 1) + 8 * (lane & 1);
   __syncthreads();
 
   f32x16 acc[N::kAgpr], accv[N::kAcc > N::kAgpr ? N::kAcc - N::kAgpr : 1];
@@ -236,7 +266,7 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
       tv[q] = *reinterpret_cast<const f32x4*>(a.target + (pv ? p : n - 1) * out + r + 4 * h);
     }
 #pragma unroll
-    for (int c = 0; c < KC0; ++c) bx[c] = c < a.kc0 ? nx[c] : half8{};
+    for (int c = 0; c < KC0; ++c) bx[c] = c < a.kc0 && pv ? nx[c] : half8{};  // points past n: no input, no gradient
     if (tile + NW < t_end) load_x(tile + NW, nx);
 
     // The next stage's fragments are read while this one computes (the wave is
@@ -250,8 +280,19 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
     };
     fetch(0);
 
-    // ---- forward
     half8 b[D][KC];
+    // g's slot s, and layer l's input h_{l-1} (two buffers), point-major into the
+    // scratch; the wave's own LDS accesses stay in order
+    auto put_g = [&](int s, const half8& v) { *(lds_h8*)(tg + ((put0 + opaque_zero()) ^ (32 * s))) = v; };
+    auto put_h = [&](int l) {
+      const uint32_t put = put0 + opaque_zero();
+#pragma unroll
+      for (int s = 0; s < (KC > KC0 ? KC : KC0); ++s)
+        if (s < (l == 0 ? KC0 : KC))
+          *(lds_h8*)(tg + (put ^ (32 * s)) + (1 + (l & 1)) * N::kTr) = l == 0 ? bx[s < KC0 ? s : 0] : b[l > 0 ? l - 1 : 0][s < KC ? s : 0];
+    };
+
+    // ---- forward
     auto bias = [&](int base) {
       f32x16 v;
 #pragma unroll
@@ -284,6 +325,7 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
     half8 g[KC];
     {
       fetch(D + 1);
+      put_h(D);
       f32x16 y = bias(D * H);
 #pragma unroll
       for (int c = 0; c < KC; ++c)
@@ -298,47 +340,27 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
           g[0][4 * hi + j] = half_t(d + d);
         }
       }
+      put_g(0, g[0]);
     }
     // ---- backward
 #pragma unroll
     for (int l = D; l >= 0; --l) {
       fetch(2 * D + 2 - l);
-      // g_l as K = points operands (and db), block by block; then this block's row of dW_l
-      half8 ht[MT > MTI ? MT : MTI][2];      // the layer's input likewise
+      // back as K = points operands.  Moved, not multiplied by a 0/1 selection: an
+      // infinity or a NaN of one feature must not reach the others.
+      const uint32_t get = get0 + opaque_zero();
+      half8 ht[MT > MTI ? MT : MTI][2], gt[MT][2];
 #pragma unroll
-      for (int t = 0; t < (l == 0 ? MTI : MT); ++t) {
-        f32x16 d = {};
-        if (l == 0) {
-          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(bx[2 * t < KC0 ? 2 * t : 0], nat0, d, 0, 0, 0);
-          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(bx[2 * t + 1 < KC0 ? 2 * t + 1 : 0], nat1, d, 0, 0, 0);
-        } else {
-          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[l > 0 ? l - 1 : 0][2 * t < KC ? 2 * t : 0], sel0, d, 0, 0, 0);
-          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[l > 0 ? l - 1 : 0][2 * t + 1 < KC ? 2 * t + 1 : 0], sel1, d, 0, 0, 0);
-        }
-        ht[t][0] = tp2_half(d, 0);
-        ht[t][1] = tp2_half(d, 1);
-      }
+      for (int t = 0; t < (l == 0 ? MTI : MT); ++t)
 #pragma unroll
-      for (int o = 0; o < (l == D ? 1 : MT); ++o) {
-        f32x16 d = {};
-        d = __builtin_amdgcn_mfma_f32_32x32x16_f16(g[2 * o], sel0, d, 0, 0, 0);
-        if (l < D) d = __builtin_amdgcn_mfma_f32_32x32x16_f16(g[2 * o + 1], sel1, d, 0, 0, 0);
-        const half8 g0 = tp2_half(d, 0), g1 = tp2_half(d, 1);
-        db[l * MT + o] = tp2_sum(g1, tp2_sum(g0, db[l * MT + o]));
+        for (int ks = 0; ks < 2; ++ks) ht[t][ks] = fused_points(tg + (get ^ (64 * t)) + (1 + (l & 1)) * N::kTr + 16 * ks * 128);
 #pragma unroll
-        for (int t = 0; t < (l == 0 ? MTI : MT); ++t) {
-          const int k = N::dw(l) + o * (l == 0 ? MTI : MT) + t;
-          if (k < N::kAgpr) {
-            fused_dw(acc[k < N::kAgpr ? k : 0], g0, ht[t][0], g1, ht[t][1]);
-          } else {
-            f32x16& v = accv[k < N::kAgpr ? 0 : k - N::kAgpr];
-            v = __builtin_amdgcn_mfma_f32_32x32x16_f16(g0, ht[t][0], v, 0, 0, 0);
-            v = __builtin_amdgcn_mfma_f32_32x32x16_f16(g1, ht[t][1], v, 0, 0, 0);
-          }
-        }
-      }
+      for (int o = 0; o < (l == D ? 1 : MT); ++o)  // (the head's rows past 16 are whatever slot 1 holds: never stored)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) gt[o][ks] = fused_points(tg + (get ^ (64 * o)) + 16 * ks * 128);
+      f32x16 d[MT];
       if (l > 0) {
-        f32x16 d[MT];
+        put_h(l - 1);
 #pragma unroll
         for (int t = 0; t < MT; ++t) d[t] = f32x16{};
 #pragma unroll
@@ -346,11 +368,34 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
 #pragma unroll
           for (int t = 0; t < MT; ++t)
             d[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wb[(2 * D + 1 - l) & 1][t * (l == D ? 1 : KC) + c], g[c], d[t], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // dW_l and db, and between their products g_{l-1}
+      auto mask = [&](int s) {
+        g[s] = fused_mask(tp2_half(d[s / 2], s & 1), b[l > 0 ? l - 1 : 0][s]);
+        put_g(s, g[s]);
+      };
+      constexpr int kPairs = MT * (MT > MTI ? MT : MTI);
 #pragma unroll
-        for (int s = 0; s < KC; ++s) {
-          const half8 hv = b[l > 0 ? l - 1 : 0][s];
-          g[s] = fused_mask(tp2_half(d[s / 2], s & 1), hv);
+      for (int i = 0; i < kPairs; ++i) {
+        const int mi = l == 0 ? MTI : MT, o = i / mi, t = i % mi;
+        if (o < (l == D ? 1 : MT)) {
+          if (t == 0) db[l * MT + o] = tp2_sum(gt[o][1], tp2_sum(gt[o][0], db[l * MT + o]));
+          const int k = N::dw(l) + o * mi + t;
+          if (k < N::kAgpr) {
+            fused_dw(acc[k < N::kAgpr ? k : 0], gt[o][0], ht[t][0], gt[o][1], ht[t][1]);
+          } else {
+            f32x16& v = accv[k < N::kAgpr ? 0 : k - N::kAgpr];
+            v = __builtin_amdgcn_mfma_f32_32x32x16_f16(gt[o][0], ht[t][0], v, 0, 0, 0);
+            v = __builtin_amdgcn_mfma_f32_32x32x16_f16(gt[o][1], ht[t][1], v, 0, 0, 0);
+          }
         }
+        if (l > 0 && i < KC) mask(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (l > 0) {
+#pragma unroll
+        for (int s = kPairs; s < KC; ++s) mask(s);
       }
     }
     fused_dw_done(acc);
@@ -364,7 +409,7 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
 #pragma unroll
   for (int i = 0; i <= D * MT; ++i) {
     const float v = db[i] + __shfl_xor(db[i], 32, 64);
-    if (h == 0) s_db[wave][32 * i + col] = v;
+    if (h == 0) s_db[wave][32 * i + hidden_slot_feature(col)] = v;  // lane col summed position col of its block
   }
   f32x4* const red = reinterpret_cast<f32x4*>(smem);  // [block][wave][4][64]
 #pragma unroll
@@ -397,7 +442,9 @@ __global__ __launch_bounds__(64 * fused_waves(MT), 1) void train_fused_kernel(Tr
         for (int w = 1; w < NW; ++w) s += red[((wave * NW + w) * 4 + q) * 64 + lane];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const int o = 32 * (r / mi) + 8 * q + 4 * h + j, i = 32 * (r % mi) + col;
+          // positions to features: g and h in the hidden order, x in its own
+          const int o = hidden_slot_feature(32 * (r / mi) + 8 * q + 4 * h + j);
+          const int i = l == 0 ? 32 * (r % mi) + col : hidden_slot_feature(32 * (r % mi) + col);
           if (o < ow && i < iw) dst[int64_t(o) * iw + i] = s[j];
         }
       }

@@ -218,3 +218,52 @@ def test_narrow_head_rows(inputs):
     dw, ref = grads[-1][0].cpu().double().numpy(), ref_grads[-1][0]
     rows = np.linalg.norm(dw - ref, axis=1) / np.linalg.norm(ref, axis=1)
     assert (rows <= 1e-2).all(), f"head rows off by {np.round(rows, 4)}"
+
+
+def _non_finite_reference(x, t, layers):
+    """The step with the kernels' treatment of infinities and NaN: ReLU maps a NaN to 0, activations and gradients are
+    rounded to fp16 (past 65504: infinite), a gradient is masked by selection; the products are IEEE's."""
+    with np.errstate(all="ignore"):
+        h = [x.astype(np.float64)]
+        for i, (w, b) in enumerate(layers):
+            z = (h[-1] @ w.astype(np.float64).T + b).astype(np.float32)
+            if i + 1 < len(layers):
+                h.append(np.fmax(z.astype(np.float16), np.float16(0)).astype(np.float64))
+        g = (2 * (z - t)).astype(np.float16).astype(np.float64)
+        grads = []
+        for l in range(len(layers) - 1, -1, -1):
+            grads.insert(0, (g.T @ h[l], g.sum(0)))
+            if l:
+                g = np.where(h[l] > 0, (g @ layers[l][0].astype(np.float64)).astype(np.float16).astype(np.float64), 0.0)
+        return [(dw / t.size, db / t.size) for dw, db in grads]
+
+
+@pytest.mark.parametrize("n", [70, 100])  # the last tile: 6 points; 4
+@pytest.mark.parametrize("dims", [[16, 64, 8], [64, 32, 32, 8], [32, 64, 64, 16], [64] + [64] * 4 + [16]])
+@pytest.mark.parametrize("where,value", [
+    ("target", float("nan")), ("target", float("inf")), ("target", 1e5),  # 1e5: the gradient overflows fp16
+    ("x", float("nan")), ("x", float("inf")), ("x", 60000.0),             # 60000: activations overflow
+    ("last x", float("inf")), ("last x", 60000.0),                        # in the row that ends a partial tile
+])
+def test_narrow_chains_keep_non_finite_values_apart(dims, n, where, value):
+    """One non-finite value reaches the gradient entries it has a part in and no others: the same entries are finite as
+    in the reference, within 1e-2 of their norm."""
+    g = torch.Generator().manual_seed(len(dims))
+    layers = [(((torch.rand(dims[i + 1], dims[i], generator=g) * 2 - 1) * (6.0 / dims[i]) ** 0.5).half().float(),
+               torch.randn(dims[i + 1], generator=g) * 0.1) for i in range(len(dims) - 1)]
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, dims[0], generator=g).half()
+    t = torch.randn(n, dims[-1], generator=g)
+    if where == "target":
+        t[5, 3] = value
+    else:
+        x[7 if where == "x" else n - 1, 5] = value
+    _, grads = rdv.mse_backward(_chain(layers), x.cuda(), t.cuda())
+    ref = _non_finite_reference(x.numpy(), t.numpy(), [(w.numpy(), b.numpy()) for w, b in layers])
+    for l, (got, want) in enumerate(zip(grads, ref)):
+        for a, b, what in zip(got, want, ("dW", "db")):
+            a = a.cpu().double().numpy()
+            finite = np.isfinite(b)
+            assert (np.isfinite(a) == finite).all(), f"layer {l} {what}: {(np.isfinite(a) != finite).sum()} entries"
+            err = np.linalg.norm(a[finite] - b[finite])
+            assert err <= 1e-2 * np.linalg.norm(b[finite]), f"layer {l} {what}: {err}"
