@@ -64,6 +64,7 @@ struct LinearGemmArgs {
   const float* bias;
   float* y;
   int64_t rows, row_tiles;
+  int64_t block0;  // this launch's first block
   int in, out, col_tiles;
   int wkind, relu;
 };
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_gemm_kernel(LinearGemmArgs 
   const int r = lane & 15, q = lane >> 4;
   // Blocks of one XCD (consecutive multiples of 8) take the column tiles of a
   // row tile one after the other, so its x rows are read from HBM once.
-  const int64_t b = blockIdx.x;
+  const int64_t b = a.block0 + blockIdx.x;
   const int ct = int((b >> 3) % a.col_tiles);
   const int64_t rt = ((b >> 3) / a.col_tiles) * 8 + (b & 7);
   if (rt >= a.row_tiles) return;
@@ -302,15 +303,20 @@ int launch_linear_gemm_t(const LinearGemmArgs& a0, hipStream_t stream) {
   a.row_tiles = (a.rows + BM - 1) / BM;
   a.col_tiles = (a.out + BN - 1) / BN;
   const int64_t grid = (a.row_tiles + 7) / 8 * 8 * a.col_tiles;
-  if (grid > 0x7fffffff) return fail(RDV_ERR_UNSUPPORTED, "grid too large");
   static bool attr = false;
   if (!attr) {
     RDV_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_gemm_kernel<F16, TILED, NW, WM, WN>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kBytes));
     attr = true;
   }
-  linear_gemm_kernel<F16, TILED, NW, WM, WN><<<dim3(unsigned(grid)), dim3(64 * NW), kBytes, stream>>>(a);
-  RDV_HIP_TRY(hipGetLastError());
+  // A launch takes at most 2^32 - 1 threads (HIP keeps their count in 32 bits and runs
+  // what is left of a larger one without an error): 1.07e9 rows of the smallest tile.
+  constexpr int64_t kMaxBlocks = 0xffffffffLL / (64 * NW) / 8 * 8;  // whole XCD rounds
+  for (a.block0 = 0; a.block0 < grid; a.block0 += kMaxBlocks) {
+    const int64_t blocks = std::min(grid - a.block0, kMaxBlocks);
+    linear_gemm_kernel<F16, TILED, NW, WM, WN><<<dim3(unsigned(blocks)), dim3(64 * NW), kBytes, stream>>>(a);
+    RDV_HIP_TRY(hipGetLastError());
+  }
   return RDV_OK;
 }
 
@@ -396,7 +402,7 @@ int launch_linear_op(const rdv_linear_op_desc& d, const float* x, const void* w,
       cost = c;
     }
   }
-  const LinearGemmArgs a = {x, w, bias, y, d.rows, 0, d.in_features, d.out_features, 0, d.wkind, d.relu ? 1 : 0};
+  const LinearGemmArgs a = {x, w, bias, y, d.rows, 0, 0, d.in_features, d.out_features, 0, d.wkind, d.relu ? 1 : 0};
   if (!f16) return launch_linear_gemm<false, false>(best, a, stream);
   if (d.wkind == RDV_WKIND_F16_TILED16 && reinterpret_cast<uintptr_t>(w) % 16 == 0)
     return launch_linear_gemm<true, true>(best, a, stream);

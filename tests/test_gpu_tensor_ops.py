@@ -384,3 +384,21 @@ def test_direct_conv_shape_errors():
                                     torch.zeros(16).cuda(), 16, 6)                          # W % 8
     with pytest.raises(AssertionError):
         rdv.Conv2DTensorOpSimple3x3(x, torch.zeros(5, 5, 16, 16).cuda(), torch.zeros(16).cuda(), 8, 8)  # not 3x3
+
+
+@pytest.mark.parametrize("rows,inf,outf", [((1 << 30) + 33, 8, 4), (1, 8, (1 << 26) + 32)])
+def test_more_threads_than_one_launch_takes(rows, inf, outf):
+    """Row and output counts whose tiles are more than 2^32 - 1 threads (51 GB of x and y; 2.4 GB of W): every output
+    against torch's product, 1e-5 for sums of 8 terms of size 1."""
+    g = torch.Generator(device="cuda").manual_seed(inf)
+    x = torch.rand(rows, inf, generator=g, device="cuda")
+    W = torch.rand(outf, inf, generator=g, device="cuda")
+    b = torch.rand(outf, generator=g, device="cuda")
+    y = torch.full((rows, outf), -1.0, device="cuda")
+    assert _raw_linear(x, W, b, y, rows, inf, outf, _lib.PREC_F32, _lib.WKIND_F32) == 0, _lib.last_error()
+    step = 1 << 26
+    for r in range(0, rows, step):
+        for o in range(0, outf, step):
+            ref = torch.addmm(b[o:o + step], x[r:r + step], W[o:o + step].t())
+            err = (y[r:r + step, o:o + step] - ref).abs().max().item()
+            assert err <= 1e-5, f"rows {r}.., outputs {o}..: off by {err}"
