@@ -14,7 +14,8 @@
 // at dispatch, like Small and Mine), fp16 [out, in] (Simple's pre-cast copy) or
 // fp16 [out/16][in/16][16 k][16 n] tiles (Fast's pre-tiled copy, nn.py:472-490).
 //
-// linear_gemm_kernel (below) serves every shape; relu_op_kernel streams.
+// linear_gemm_kernel (below) serves most shapes, linear_stream_kernel large fp32
+// products over few columns; relu_op_kernel streams.
 #include <algorithm>
 
 #include "rdv_common.h"
@@ -320,6 +321,128 @@ int launch_linear_gemm_t(const LinearGemmArgs& a0, hipStream_t stream) {
   return RDV_OK;
 }
 
+// -------------------------------------------------- few columns, many rows (fp32)
+// A persistent block of 4 waves owns up to 128 outputs: it stages their weights and
+// biases in LDS once, as the A fragments of v_mfma_f32_16x16x4f32 (slot (t, c, lane):
+// W[o0 + 16 t + lane % 16][16 c + 4 (lane / 16) ..]), then its waves walk 32-row tiles
+// with a grid stride and no barrier, the next tile's x loaded (16 bytes a lane)
+// while this one is computed.  The products and their order are linear_gemm_kernel's.
+//
+// linear_gemm_kernel stages whole steps of 32 columns and its blocks load, compute and
+// store in turn; with one or two steps there is little to overlap, and up to half of
+// it is padding.  Bound: HBM.  Measured, gemm and this kernel: 262,144 x 8 -> 128 37.7 and
+// 24.7 us, 65,536 x 48 -> 512 56 and 42, 65,536 x 16 -> 1024 76 and 47, 4,194,304 x 8 -> 4 111
+// and 58.
+constexpr int kLsThreads = 256, kLsWaves = 4, kLsOutputs = 128, kLsRows = 32;  // rows per wave and tile
+
+struct LinearStreamArgs {
+  const float* x;
+  const float* w;
+  const float* bias;
+  float* y;
+  int64_t rows, tasks;  // tasks: tiles of kLsWaves * kLsRows rows
+  int in, out, relu;
+  int ob, n_ob;         // outputs per block (a multiple of 16), blocks of outputs
+};
+
+template <int NKC, int G>  // chunks of 16 columns, tiles of 16 outputs stored together
+__global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamArgs a) {
+  extern __shared__ f32x4 lo_smem[];
+  const int nt = a.ob / 16;
+  f32x4* const sw = lo_smem;                     // [nt][NKC][64]
+  f32x4* const sb = lo_smem + nt * NKC * 64;     // [ob / 4]
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // blocks of the same rows are neighbours, so their x re-reads hit the shared cache
+  const int o0 = int(blockIdx.x % unsigned(a.n_ob)) * a.ob;
+  const int64_t stride = gridDim.x / unsigned(a.n_ob);
+  const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = threadIdx.x; s < nt * NKC * 64; s += kLsThreads) {
+    const int o = o0 + 16 * (s / (NKC * 64)) + (s & 15);
+    const int k = 16 * ((s >> 6) % NKC) + 4 * ((s & 63) >> 4);
+    sw[s] = o < a.out && k < a.in ? *reinterpret_cast<const f32x4*>(a.w + int64_t(o) * a.in + k) : zero4;
+  }
+  for (int i = threadIdx.x; i < a.ob; i += kLsThreads) reinterpret_cast<float*>(sb)[i] = o0 + i < a.out ? a.bias[o0 + i] : 0.0f;
+  __syncthreads();
+
+  f32x4 raw[2][NKC], xf[2][NKC];
+  // rows clamped into range (their results are not stored), columns past `in` to
+  // column 0 (zeroed on use): every load is in bounds
+  auto load = [&](int64_t task) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t row = (task * kLsWaves + wave) * kLsRows + 16 * h + r;
+      const float* xr = a.x + (row < a.rows ? row : a.rows - 1) * a.in;
+#pragma unroll
+      for (int c = 0; c < NKC; ++c) raw[h][c] = *reinterpret_cast<const f32x4*>(xr + (16 * c + 4 * q < a.in ? 16 * c + 4 * q : 0));
+    }
+  };
+  int64_t task = blockIdx.x / unsigned(a.n_ob);
+  if (task < a.tasks) load(task);
+  for (; task < a.tasks; task += stride) {
+#pragma unroll
+    for (int c = 0; c < NKC; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) xf[h][c] = 16 * c + 4 * q < a.in ? raw[h][c] : zero4;
+    load(task + stride < a.tasks ? task + stride : a.tasks - 1);
+    const int64_t row0 = (task * kLsWaves + wave) * kLsRows + r;
+    float* const y0 = a.y + row0 * a.out + o0 + 4 * q;
+    // G tiles of 16 outputs at a time, their stores together: 2 make whole 128-byte lines
+    // of y; for a y past the caches 8, whole rows of the block (1,048,576 x 48 -> 256 404 us
+    // with 2, 367 with 8; 65,536 x 48 -> 512 42.1 and 43.4).
+    for (int t0 = 0; t0 < nt; t0 += G) {
+      f32x4 acc[G][2];
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        const int t = t0 + u < nt ? t0 + u : nt - 1;
+        acc[u][0] = acc[u][1] = sb[4 * t + q];
+#pragma unroll
+        for (int c = 0; c < NKC; ++c) {
+          const f32x4 wv = sw[(t * NKC + c) * 64 + lane];
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) acc[u][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[k], xf[h][c][k], acc[u][h], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (row0 + 16 * h < a.rows) {
+#pragma unroll
+          for (int u = 0; u < G; ++u) {
+            if (t0 + u < nt && o0 + 16 * (t0 + u) + 4 * q < a.out) {
+              if (a.relu) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[u][h][j] = fmaxf(acc[u][h][j], 0.0f);
+              }
+              *reinterpret_cast<f32x4*>(y0 + int64_t(16 * h) * a.out + 16 * (t0 + u)) = acc[u][h];
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int NKC, int G>
+int launch_linear_stream_t(const LinearStreamArgs& a, int cu, hipStream_t stream) {
+  const size_t lds = size_t(a.ob / 16) * NKC * 1024 + size_t(a.ob) * 4;  // at most 32.5 KiB
+  int occ = 0;
+  RDV_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, linear_stream_kernel<NKC, G>, kLsThreads, lds));
+  const int64_t slots = int64_t(cu) * std::max(occ, 1);
+  const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(a.tasks, (slots + a.n_ob - 1) / a.n_ob));
+  linear_stream_kernel<NKC, G><<<dim3(unsigned(groups * a.n_ob)), dim3(kLsThreads), lds, stream>>>(a);
+  RDV_HIP_TRY(hipGetLastError());
+  return RDV_OK;
+}
+
+template <int NKC>
+int launch_linear_stream(const LinearStreamArgs& a, int cu, hipStream_t stream) {
+  if (a.ob == kLsOutputs && a.rows * a.out >= int64_t(1) << 27) return launch_linear_stream_t<NKC, 8>(a, cu, stream);
+  return launch_linear_stream_t<NKC, 2>(a, cu, stream);
+}
+
 __global__ __launch_bounds__(256) void relu_op_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t n) {
   const int64_t n4 = n >> 2;
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
@@ -386,6 +509,26 @@ int launch_linear_op(const rdv_linear_op_desc& d, const float* x, const void* w,
   DeviceInfo dev;
   if (int rc = device_info(&dev)) return rc;
   const bool f16 = d.precision == RDV_PREC_F16;
+  if (!f16 && d.in_features <= 64) {
+    // linear_stream_kernel where its blocks fill the chip, so many per CU that it is the
+    // faster of the two (us, linear_gemm_kernel and this one, just below and at the line):
+    // up to 16 columns 2 (32,768 x 8 -> 128, 1 per CU, 7.7 and 7.0; 65,536 x 8 -> 128 12.3 and
+    // 9.7), to 32 4 (65,536 x 32 -> 128, 2, 12.8 and 12.9; 65,536 x 24 -> 256 21.5 and 19.6),
+    // to 48 2 (32,768 x 48 -> 128, 1, 10.4 and 10.5; 65,536 x 40 -> 128 17.9 and 15.8), to 64 8
+    // (32,768 x 64 -> 512, 4, 29.4 and 30.9; 65,536 x 64 -> 512 55.1 and 51.5).
+    LinearStreamArgs a = {x, static_cast<const float*>(w), bias, y, d.rows, 0, d.in_features, d.out_features, d.relu ? 1 : 0, 0, 0};
+    a.tasks = (d.rows + kLsWaves * kLsRows - 1) / (kLsWaves * kLsRows);
+    a.ob = std::min(kLsOutputs, (d.out_features + 15) / 16 * 16);
+    a.n_ob = (d.out_features + a.ob - 1) / a.ob;
+    const int chunks = (d.in_features + 15) / 16;
+    const int per_cu = chunks == 4 ? 8 : chunks == 2 ? 4 : 2;
+    if (a.tasks * a.n_ob >= int64_t(per_cu) * dev.cu_count) {
+      if (chunks == 1) return launch_linear_stream<1>(a, dev.cu_count, stream);
+      if (chunks == 2) return launch_linear_stream<2>(a, dev.cu_count, stream);
+      if (chunks == 3) return launch_linear_stream<3>(a, dev.cu_count, stream);
+      return launch_linear_stream<4>(a, dev.cu_count, stream);
+    }
+  }
   // The tile whose busiest CU has the least work: tiles per CU, rounded up, times
   // a tile's area over its efficiency.  Large products take the 256 x 256 tile,
   // small ones the one that still gives every CU a block, and none pays for a

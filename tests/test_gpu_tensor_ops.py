@@ -399,6 +399,32 @@ def test_more_threads_than_one_launch_takes(rows, inf, outf):
     step = 1 << 26
     for r in range(0, rows, step):
         for o in range(0, outf, step):
-            ref = torch.addmm(b[o:o + step], x[r:r + step], W[o:o + step].t())
+            ref = b[o:o + step].expand(min(step, rows - r), -1).clone()
+            for k in range(inf):
+                ref.addcmul_(x[r:r + step, k:k + 1], W[o:o + step, k])
             err = (y[r:r + step, o:o + step] - ref).abs().max().item()
             assert err <= 1e-5, f"rows {r}.., outputs {o}..: off by {err}"
+
+
+@pytest.mark.parametrize("rows,inf,outf", [
+    (65537, 8, 4), (65569, 16, 36), (16385, 12 * 2, 1000), (131073, 32, 72), (65535, 40, 132), (32801, 48, 516),
+    (65599, 56, 512), (262145, 64, 20), ((1 << 20) + 1, 16, 128),  # the last: y of 2^27 elements and more
+])
+@pytest.mark.parametrize("relu", [False, True])
+def test_linear_op_few_columns(rows, inf, outf, relu):
+    """fp32 products of up to 64 columns at row counts that take the streaming kernel, ragged in every dimension, within
+    twice the bound of any fp32 summation order; nothing past the last row is written."""
+    g = torch.Generator(device="cuda").manual_seed(rows + inf)
+    x = torch.randn(rows, inf, generator=g, device="cuda")
+    W = torch.randn(outf, inf, generator=g, device="cuda") / inf ** 0.5
+    b = torch.randn(outf, generator=g, device="cuda")
+    y = torch.full(((rows + 2) * outf,), 12345.0, device="cuda")
+    assert _raw_linear(x, W, b, y, rows, inf, outf, _lib.PREC_F32, _lib.WKIND_F32, relu) == 0, _lib.last_error()
+    assert bool((y[rows * outf:] == 12345.0).all()), "kernel wrote past the last row"
+    u, k = 2.0 ** -24, inf + 2
+    for r in range(0, rows, 1 << 18):
+        xr = x[r:r + (1 << 18)].double()
+        ref = torch.addmm(b.double(), xr, W.double().t())
+        bound = 2 * k * u / (1 - k * u) * torch.addmm(b.double().abs(), xr.abs(), W.double().abs().t())
+        got = y[: rows * outf].view(rows, outf)[r:r + (1 << 18)].double()
+        assert bool(((got - (ref.clamp_min(0.0) if relu else ref)).abs() <= bound).all()), f"rows {r}.."
