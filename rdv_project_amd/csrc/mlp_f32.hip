@@ -275,7 +275,11 @@ __device__ __forceinline__ void chain_f32_body(const ChainF32Args& ga, float* sm
   const int64_t t_begin = int64_t(blockIdx.x) * per_block;
   const int64_t t_end = t_begin + per_block < ga.tiles ? t_begin + per_block : ga.tiles;
   const int D = ga.enc_d, in0 = ga.layer[0].in_w;
-  // act[i] of lane (q, m): feature 4 i + q of row m of the tile, zero past in0
+  // act[i] of lane (q, m): feature 4 i + q of row m of the tile; past in0 the row's
+  // last one, zeroed by mask_raw (the wide kernel has no registers to put that off).
+  // Loads only, four to a branch: a select beside each one waited for it, a memory
+  // latency per four features of every tile (262,144 rows of 64 -> 64 -> 64 -> 16: 303 us,
+  // now 61; 164 on the vector ALUs).
   auto load_raw = [&](int64_t tile, float (&act)[4 * MT]) {
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));  // per-tile masks and addresses, as in chain_layer_m
@@ -283,14 +287,32 @@ __device__ __forceinline__ void chain_f32_body(const ChainF32Args& ga, float* sm
     const int64_t r = tile * 16 + (lane & 15);
     const float* xr = ga.x + (ga.row0 + (r < ga.nrows ? r : ga.nrows - 1)) * D;
 #pragma unroll
-    for (int i = 0; i < 4 * MT; ++i) {
-      act[i] = 0.0f;
-      if (4 * i < in0) {
+    for (int c = 0; c < MT; ++c) {
+      if (16 * c < in0) {
         chain_branch();
-        const float v = xr[4 * i + q < in0 ? 4 * i + q : 0];
-        act[i] = 4 * i + q < in0 ? v : 0.0f;
+#pragma unroll
+        for (int i = 4 * c; i < 4 * c + 4; ++i) act[i] = xr[min(4 * i + q, in0 - 1)];
+        if (MT > 4 && 16 * c + 16 > in0) {
+#pragma unroll
+          for (int i = 4 * c; i < 4 * c + 4; ++i) act[i] = 4 * i + q < in0 ? act[i] : 0.0f;
+        }
+      } else if (MT > 4) {
+#pragma unroll
+        for (int i = 4 * c; i < 4 * c + 4; ++i) act[i] = 0.0f;
       }
     }
+  };
+  auto mask_raw = [&](float (&act)[4 * MT]) {
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
+    const int q = lane >> 4;
+#pragma unroll
+    for (int c = 0; c < MT; ++c)
+      if (16 * c + 16 > in0) {
+        chain_branch();
+#pragma unroll
+        for (int i = 4 * c; i < 4 * c + 4; ++i) act[i] = 4 * i + q < in0 ? act[i] : 0.0f;
+      }
   };
   const bool freq = ga.encoding == RDV_ENC_FREQ;
   float act[4 * MT] = {};
@@ -348,6 +370,8 @@ __device__ __forceinline__ void chain_f32_body(const ChainF32Args& ga, float* sm
 #pragma unroll
         for (int k = 0; k < 4 * MT; ++k) act[k] = k == i ? v : act[k];
       }
+    } else if (MT == 4) {
+      mask_raw(act);
     }
 #pragma nounroll
     for (int l = 0; l < L; ++l) {
