@@ -29,7 +29,7 @@ struct ChainStageSlot {
   const float* src;  // first element of the slot's first row
   int dst;           // LDS float offset of that row
   int stride;        // LDS row stride in floats
-  int iw;            // columns; pieces past iw are zero
+  int iw;            // columns; past them kChainPad
   int units;         // pieces of this slot (<= threads per block)
   float inv_kq;      // 1 / pieces per row, pieces per row = ceil(iw / 4)
   int vec_f16;       // bit 0: rows of whole 16-byte pieces, 16-byte aligned; bit 1: round the values to fp16
@@ -80,8 +80,12 @@ __device__ __forceinline__ float chain_input(const ChainF32Args& a, const float*
   return r < D ? sinpif(t) : cospif(t);
 }
 
+// What stands for a weight past a layer's last column: times the +0 its input is
+// padded with it leaves every sum as it is, a sum of -0 too (+0 would make that +0).
+constexpr float kChainPad = -0.0f;
+
 // Weights W[row][16 c + 4 s + q], s = 0..3, of chunk c for this lane: from LDS
-// (columns past the layer's width are staged as zeros up to a multiple of 4; the
+// (columns past the layer's width are staged as kChainPad up to a multiple of 4; the
 // callers ask for no later ones), or from the layer's own rows.
 template <bool LDSW>
 __device__ __forceinline__ float chain_weight(const float* w, int row, int k, int iw, bool f16) {
@@ -90,7 +94,7 @@ __device__ __forceinline__ float chain_weight(const float* w, int row, int k, in
   } else {
     float v = w[row + (k < iw ? k : 0)];
     if (f16) v = float(half_t(v));
-    return k < iw ? v : 0.0f;
+    return k < iw ? v : kChainPad;
   }
 }
 
@@ -340,7 +344,7 @@ __device__ __forceinline__ void chain_f32_body(const ChainF32Args& ga, float* sm
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[k][j] = src[e + min(j, last)];
 #pragma unroll
-        for (int j = 1; j < 4; ++j) v[k][j] = j <= last ? v[k][j] : 0.0f;
+        for (int j = 1; j < 4; ++j) v[k][j] = j <= last ? v[k][j] : kChainPad;
       }
     }
 #pragma unroll

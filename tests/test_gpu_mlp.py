@@ -484,3 +484,15 @@ def test_dispatch_map_evaluator_and_deferred_kwargs():
     assert torch.equal(y, want)
     with pytest.raises(RuntimeError):
         rdv.Deferred("scale").resolve()  # unbound again after the call
+
+
+@pytest.mark.parametrize("n", [5, 9000])
+@pytest.mark.parametrize("dims", [[1, 3], [3, 5], [7, 3], [33, 6], [101, 5], [255, 130]])
+def test_f32_chain_keeps_negative_zero(dims, n):
+    """Every product rounds to -0 on top of a sum of -0: the outputs are -0 to the sign bit, as of a loop of fused
+    multiply-adds, at widths that the 4-wide matrix products pad."""
+    g = WL.gen(3)
+    w = torch.rand(dims[1], dims[0], generator=g) * 1e-30 + 1e-31
+    x = -torch.rand(n, dims[0], generator=g) * 1e-30 - 1e-31
+    y = _chain([(w, torch.full((dims[1],), -0.0))], ["none"], f16=[False])(x.cuda()).as_tensor("torch").cpu()
+    assert bool((y == 0).all()) and bool(torch.signbit(y).all()), f"{int((~torch.signbit(y)).sum())} of {y.numel()} are +0"
