@@ -45,8 +45,8 @@ namespace rdv {
 // the chain plus whatever the slowest lane has to do between two points.  Three things keep
 // that short (512 x 512 rays, 16 environment samples, 5-layer 64-wide chain: 10.25 ms without
 // them, 6.99 with; 180 x 100 rays, 4 samples: 4.88 and 2.30):
-//   - a step inside a march runs by itself (vp_march_step); the state machine's other parts
-//     run when half of the wave's rays wait for them;
+//   - a step inside a march runs by itself (vp_march_step); where it pays (kVpWaitShare), the
+//     state machine's other parts run when half of the wave's rays wait for them;
 //   - a tracked ray that grazes a voxel face takes its flights without divisions or logarithms;
 //   - a launch's rays are spread over every CU, and a wave with at most 32 rays evaluates one
 //     tile a round.
@@ -628,9 +628,14 @@ struct VpGenArgs {
 };
 
 // A wave's waiting rays are served when they are at least 1 / kVpWaitShare of its
-// rays (or none marches).  512 x 512 rays, 16 environment samples each, 5-layer
-// 64-wide extinction chain: share 2 7.0 ms, 3 7.3, 4 7.3, 6 7.2; 180 x 100 rays
-// within 1% of one another.
+// rays (or none marches), in launches that fill waves of a cheap chain with rays
+// that also track environment samples: there some ray waits in nearly every round, and
+// serving it costs more than an evaluation.  512 x 512 rays, 16 environment samples
+// each, 5-layer 64-wide extinction chain: share 2 7.0 ms, 3 7.3, 4 7.3, 6 7.2.  Everywhere
+// else a ray is served when it waits: its later phases start the sooner, and a small
+// launch lasts as long as its longest ray (share 2 and at once: 400 x 400 rays without
+// environment samples, DDA, 64 x 3 2.48 and 1.80 ms; 64 x 64 rays, FREQ(6) -> 64 x 2 5.0
+// and 3.3; 400 x 400 rays, 256 x 2, 2 samples 26.1 and 20.9).
 constexpr int kVpWaitShare = 2;
 
 // One block's rays (DDA: VolumeProfileDDA's marches, a compile-time choice so that
@@ -675,26 +680,28 @@ __device__ __forceinline__ void volume_profile_body(const VpGenArgs& ga) {
   float sigma = 0.0f;
   // A block with at most 32 rays for each of its waves gives every wave its share
   // at once and evaluates one tile a round: the time is then the longest ray's
-  // rounds, and a wave that took 64 rays would leave others without any.
-  const int waves = int(blockDim.x) >> 6;
+  // rounds, and a wave that took 64 rays would leave others without any.  With exact
+  // fp32 layers the matrix cores bound a round, so one wave per SIMD takes rays (64 x
+  // 64 rays, 64 x 3: 8.7 ms with 2 per SIMD, 7.0 with 1).
+  const int waves = F32L ? min(int(blockDim.x) >> 6, 4) : int(blockDim.x) >> 6;
   const int share = (nr + waves - 1) / waves;
   const bool narrow = share <= 32;
-  if (narrow && (W64 ? lane : col) >= share) exhausted = true;
+  if (narrow && ((W64 ? lane : col) >= share || int(threadIdx.x) >> 6 >= waves)) exhausted = true;
+  const int wait = (W64 || (MT == 1 && !F32L)) && !narrow && a.es > 0 ? kVpWaitShare : 64;
   const uint64_t below = (uint64_t(1) << (W64 ? lane : col)) - 1;
   const bool owner = W64 || h == 0;  // the lane whose ballot bit stands for its ray
   for (;;) {
     // Marches step here; everything else (a march's end, a threshold, a DDA cell's
-    // exit, a tracked ray's flights, the next ray) waits until a share of the
-    // wave's rays does: that code is ten times a step's length, and with 64 rays
-    // some ray needed it in nearly every round, the others standing by.  What a
-    // ray computes does not depend on when it runs.
+    // exit, a tracked ray's flights, the next ray) may wait until a share of the
+    // wave's rays does: that code is ten times a step's length.  What a ray computes
+    // does not depend on when it runs.
     if (ray >= 0 && has && vp_march_step<DDA>(c, r, sigma, q)) {
       pending = true;
       has = false;
     }
     const int waiting = __builtin_popcountll(__builtin_amdgcn_ballot_w64(owner && !pending && (ray >= 0 || !exhausted)));
     const int marching = __builtin_popcountll(__builtin_amdgcn_ballot_w64(owner && pending));
-    while (waiting * kVpWaitShare >= waiting + marching) {  // all of the wave's rays that wait, then no more
+    while (waiting * wait >= waiting + marching) {  // all of the wave's rays that wait, then no more
       if (ray >= 0 && !pending) {
         const int state = vp_advance<DDA>(c, r, ray, has, sigma, q);
         has = false;
