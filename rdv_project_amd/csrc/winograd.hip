@@ -1081,14 +1081,16 @@ int launch_winograd3x3(const rdv_conv_desc& d, const void* x, const void* U, con
       if (chw) winograd3x3_kernel<1, true, true><<<grid, block, 0, stream>>>(a);
       else winograd3x3_kernel<1, true, false><<<grid, block, 0, stream>>>(a);
     } else {
-      winograd3x3_kernel<1, false, false><<<grid, block, 0, stream>>>(a);
+      if (chw) winograd3x3_kernel<1, false, true><<<grid, block, 0, stream>>>(a);
+      else winograd3x3_kernel<1, false, false><<<grid, block, 0, stream>>>(a);
     }
   } else {
     if (f16) {
       if (chw) winograd3x3_kernel<2, true, true><<<grid, block, 0, stream>>>(a);
       else winograd3x3_kernel<2, true, false><<<grid, block, 0, stream>>>(a);
     } else {
-      winograd3x3_kernel<2, false, false><<<grid, block, 0, stream>>>(a);
+      if (chw) winograd3x3_kernel<2, false, true><<<grid, block, 0, stream>>>(a);
+      else winograd3x3_kernel<2, false, false><<<grid, block, 0, stream>>>(a);
     }
   }
   RDV_HIP_TRY(hipGetLastError());

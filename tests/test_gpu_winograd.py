@@ -9,6 +9,7 @@ Bars:
     |y - ref| <= 2e-3 max(1, max|ref|) + 1e-2 |ref| (the fp16 rounding of the
     U and V operands is relative to their magnitude, so the absolute term
     scales with the output's range)."""
+import ctypes as C
 import glob
 import os
 
@@ -266,3 +267,27 @@ def test_strip_kernel_odd_channels(cin, dtype):
     w = rng.normal(0, 0.2, (3, 3, cin, 16)).astype(np.float32)
     y = _run(x, w, None, _lib.LAYOUT_HWC, dtype, _lib.LAYOUT_HWC, _lib.DTYPE_F32, False)
     _check_close(y[0], O.winograd_conv(x[0], w, np.zeros(16, np.float32)), f"cin {cin}")
+
+
+@pytest.mark.parametrize("cin", [3, 40])
+@pytest.mark.parametrize("layout", [_lib.LAYOUT_CHW, _lib.LAYOUT_HWC])
+@pytest.mark.parametrize("dtype", [_lib.DTYPE_F32, _lib.DTYPE_F16])
+def test_unaligned_image(cin, layout, dtype):
+    """An image two bytes past a 4-byte boundary is read in its own layout."""
+    rng = np.random.default_rng(cin)
+    x = rng.uniform(-1, 1, (6, 34, cin)).astype(np.float16).astype(np.float32)
+    w = rng.normal(0, 0.2, (3, 3, cin, 16)).astype(np.float32)
+    xt = torch.tensor(x.transpose(2, 0, 1) if layout == _lib.LAYOUT_CHW else x).contiguous()
+    xt = xt.to(torch.float16 if dtype == _lib.DTYPE_F16 else torch.float32)
+    raw = xt.reshape(-1).view(torch.uint8)
+    buf = torch.zeros(raw.numel() + 16, dtype=torch.uint8)
+    buf[2:2 + raw.numel()] = raw
+    buf = buf.cuda()
+    U = _conv.transform_weight(torch.tensor(w).cuda(), _lib.WLAYOUT_RSCK)
+    y = torch.full((6, 34, 16), float("nan"), device="cuda")
+    d = _conv.conv_desc(1, 6, 34, cin, 16, layout, dtype, _lib.LAYOUT_HWC, _lib.DTYPE_F32, False)
+    rc = _lib.load().rdv_winograd3x3_forward(C.byref(d), C.c_void_p(buf.data_ptr() + 2), C.c_void_p(U.data_ptr()), None,
+                                             C.c_void_p(y.data_ptr()), None)
+    torch.cuda.synchronize()
+    assert rc == 0, _lib.last_error()
+    _check_close(y.cpu().numpy(), O.winograd_conv(x, w, np.zeros(16, np.float32)), f"cin {cin}")
