@@ -1065,7 +1065,11 @@ int launch_winograd3x3(const rdv_conv_desc& d, const void* x, const void* U, con
   const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(slices)), block(256);
   // Patches of whole vectors: channels-last quartets, NCHW dwords.  The strip kernel stays for the rest (element loads).
   const uintptr_t xa = reinterpret_cast<uintptr_t>(x);
-  if (chw ? xa % 4 == 0 : d.cin % 4 == 0 && xa % (f16 ? 8 : 16) == 0) {
+  // NCHW fp32 images of more than 32 channels past the 256 MiB cache stay there too: each
+  // pixel is loaded by up to four threads, a dword at a time (1448 x 1450, 64 -> 64: 980
+  // us, strips 722; 1024 x 1026, 48 -> 48, 202 MB: 294 and 338).
+  const bool past_cache = chw && !f16 && d.cin > 32 && int64_t(d.batch) * d.H * d.W * d.cin >= int64_t(1) << 26;
+  if (chw ? xa % 4 == 0 && !past_cache : d.cin % 4 == 0 && xa % (f16 ? 8 : 16) == 0) {
 #define RDV_WG_PATCH(MODE) \
   if (d.cin <= 32) winograd3x3_patch_kernel<1, MODE><<<grid, block, 0, stream>>>(a); else winograd3x3_patch_kernel<2, MODE><<<grid, block, 0, stream>>>(a)
     if (chw && f16) { RDV_WG_PATCH(kPatchChwF16); }

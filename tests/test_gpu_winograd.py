@@ -291,3 +291,20 @@ def test_unaligned_image(cin, layout, dtype):
     torch.cuda.synchronize()
     assert rc == 0, _lib.last_error()
     _check_close(y.cpu().numpy(), O.winograd_conv(x, w, np.zeros(16, np.float32)), f"cin {cin}")
+
+
+def test_large_fp32_nchw_matches_its_crop():
+    """An NCHW fp32 image past 256 MiB takes the strip kernel: the same bits as a crop of it, which takes the patch
+    kernel, where the crop's border has no part."""
+    H, W, cin, cout, h = 1024, 1026, 64, 16, 64
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand(1, cin, H, W, generator=g, device="cuda") * 2 - 1
+    U = _conv.transform_weight(torch.randn(3, 3, cin, cout, generator=g, device="cuda") * 0.1, _lib.WLAYOUT_RSCK)
+    y = torch.full((1, cout, H, W), float("nan"), device="cuda")
+    f32, chw = _lib.DTYPE_F32, _lib.LAYOUT_CHW
+    _conv.forward(_conv.conv_desc(1, H, W, cin, cout, chw, f32, chw, f32, False), x, U, None, y)
+    for r in (0, 480, H - h):
+        yc = torch.full((1, cout, h, W), float("nan"), device="cuda")
+        _conv.forward(_conv.conv_desc(1, h, W, cin, cout, chw, f32, chw, f32, False), x[:, :, r:r + h].contiguous(), U, None, yc)
+        a, b = (0 if r == 0 else 2), (h if r == H - h else h - 2)
+        assert torch.equal(y[:, :, r + a:r + b], yc[:, :, a:b]), f"rows {r}.."
