@@ -1385,6 +1385,7 @@ __global__ __launch_bounds__(kB0Threads, 2) void train_bwd0_kernel(TrainBwdArgs 
 struct TrainPlan {
   int groups;
   int g0[RDV_MLP_MAX_LAYERS + 1];  // group k = layers [g0[k], g0[k + 1])
+  int blocks_fused;                // > 0: the step is train_fused_kernel with so many blocks
   int blocks_fwd, blocks_bwd, blocks_pair;
   bool keep[RDV_MLP_MAX_LAYERS];   // h_i stored by the forward
   int64_t wt_off[RDV_MLP_MAX_LAYERS], h_off[RDV_MLP_MAX_LAYERS], g_off, dz_off[2], dw_off[RDV_MLP_MAX_LAYERS],
@@ -1473,6 +1474,26 @@ int train_check(const rdv_mlp_desc& d, const MlpLayout& lay) {
 
 static void train_plan(const rdv_mlp_desc& d, const MlpLayout& lay, int64_t n, int cu, TrainPlan* p) {
   const int L = d.n_layers;
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t o = off;
+    off = align256(off + bytes);
+    return o;
+  };
+  // per-layer partials and the loss's, all reduced together at the end of the step
+  auto take_partials = [&](int64_t parts, int64_t loss_parts) {
+    for (int i = 0; i < L; ++i) {
+      p->dw_off[i] = take(parts * d.dims[i + 1] * d.dims[i] * 4);
+      p->db_off[i] = take(parts * d.dims[i + 1] * 4);
+    }
+    p->loss_off = take(loss_parts * 4);
+    p->total = off;
+  };
+  p->blocks_fused = train_fused_ok(d) ? train_fused_blocks(d, n, cu) : 0;
+  if (p->blocks_fused > 0) {  // one kernel, nothing else through memory
+    take_partials(p->blocks_fused, p->blocks_fused);
+    return;
+  }
   p->groups = 0;
   int l = 0;
   while (l < L) {
@@ -1489,12 +1510,6 @@ static void train_plan(const rdv_mlp_desc& d, const MlpLayout& lay, int64_t n, i
   for (int i = 0; i < RDV_MLP_MAX_LAYERS; ++i) p->keep[i] = false;
   for (int i = L - 2; i >= 1; i -= 2) p->keep[i] = true;
   for (int k = 1; k < p->groups; ++k) p->keep[p->g0[k]] = true;
-  int64_t off = 0;
-  auto take = [&](int64_t bytes) {
-    const int64_t o = off;
-    off = align256(off + bytes);
-    return o;
-  };
   int maxw = 0;
   for (int i = 0; i < L; ++i) {
     p->wt_off[i] = take(int64_t(d.dims[i] / 32 > 0 ? d.dims[i] / 32 : 1) * ((d.dims[i + 1] + 15) / 16) * 1024);
@@ -1506,17 +1521,7 @@ static void train_plan(const rdv_mlp_desc& d, const MlpLayout& lay, int64_t n, i
   p->g_off = take(rows * ((d.dims[L] + 15) / 16 * 16) * 2);
   p->dz_off[0] = take(rows * maxw * 2);
   p->dz_off[1] = take(rows * maxw * 2);
-  // per-layer partials, all reduced together at the end of the step
-  const int64_t parts = std::max(p->blocks_bwd, p->blocks_pair);
-  int64_t all = 1;  // the loss
-  for (int i = 0; i < L; ++i) {
-    p->dw_off[i] = take(parts * d.dims[i + 1] * d.dims[i] * 4);
-    p->db_off[i] = take(parts * d.dims[i + 1] * 4);
-    all += int64_t(d.dims[i + 1]) * (d.dims[i] + 1);
-  }
-  p->loss_off = take(int64_t(p->blocks_fwd) * 4);
-  take(int64_t(32) * all * 4);  // unused: keeps the workspace size, and with it what the static scratch accepts
-  p->total = off;
+  take_partials(std::max(p->blocks_bwd, p->blocks_pair), p->blocks_fwd);
 }
 
 int64_t train_workspace_bytes(const rdv_mlp_desc& d, const MlpLayout& lay, int64_t n, int cu) {
@@ -1556,17 +1561,15 @@ int launch_train_step(const rdv_mlp_desc& d, const MlpLayout& lay, const void* p
     RDV_HIP_TRY(hipGetLastError());
     return RDV_OK;
   };
-  if (train_fused_ok(d)) {
-    // one kernel for the whole step; its loss partials take the place of the
-    // gradients between backward launches, which it does not have
-    const int nb = train_fused_blocks(d, n, di.cu_count);
+  if (p.blocks_fused > 0) {  // one kernel for the whole step
+    const int nb = p.blocks_fused;
     float* parts_w[RDV_MLP_MAX_LAYERS];
     float* parts_b[RDV_MLP_MAX_LAYERS];
     for (int l = 0; l < L; ++l) {
       parts_w[l] = reinterpret_cast<float*>(ws + p.dw_off[l]);
       parts_b[l] = reinterpret_cast<float*>(ws + p.db_off[l]);
     }
-    float* lp = reinterpret_cast<float*>(ws + p.dz_off[0]);
+    float* lp = reinterpret_cast<float*>(ws + p.loss_off);
     rc = launch_train_fused(d, lay, packed, x, target, n, nb, lp, parts_w, parts_b, stream);
     if (rc == RDV_OK) rc = reduce(lp, nb, 1, loss);
     for (int l = 0; l < L && rc == RDV_OK; ++l) {

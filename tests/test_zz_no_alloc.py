@@ -94,3 +94,41 @@ def test_static_scratch_rejects_oversize_workspace():
                                        C.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert rc == _lib.RDV_ERR_WORKSPACE
     assert "static scratch" in _lib.last_error()
+
+
+@pytest.mark.parametrize("dims", [[16, 32, 8], [64] + [64] * 4 + [16]])
+def test_narrow_chains_need_their_partials_only(dims):
+    """A chain that one kernel trains keeps nothing but per-block partials: its workspace stops growing with n, a step
+    writes nothing past it, and the static scratch serves any n with the caller workspace's bits."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(len(dims))
+    m = _chain_of([(torch.randn(dims[i + 1], dims[i], generator=g) / dims[i] ** 0.5,
+                    torch.randn(dims[i + 1], generator=g) * 0.1) for i in range(len(dims) - 1)])
+    p = _chain.plan_chain(m, dims[0])
+    packed = _chain.packed_params(m, p)
+    size = [int(lib.rdv_mlp_train_workspace_bytes(C.byref(p.desc), C.c_int64(n))) for n in (1, 100, 1 << 20, 1 << 24)]
+    assert 0 < size[0] <= size[1] <= size[2] == size[3]
+    params = sum((a + 1) * b for a, b in zip(dims, dims[1:]))
+    assert size[0] <= 4 * params + 256 * 2 * len(dims) and size[3] <= _lib.TRAIN_STATIC_SCRATCH_BYTES
+    n = (1 << 20) + 5
+    x = torch.randn(n, dims[0], generator=g).half().cuda()
+    t = torch.randn(n, dims[-1], generator=g).cuda()
+    for rows in (n, 100):
+        xs, ts = x[:rows].contiguous(), t[:rows].contiguous()
+        need = int(lib.rdv_mlp_train_workspace_bytes(C.byref(p.desc), C.c_int64(rows)))
+        ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+        off = (-ws.data_ptr()) % 256
+        loss, grads = torch.full((), float("nan"), device="cuda"), _grads(p)
+        rc = lib.rdv_mlp_train_step(C.byref(p.desc), C.c_void_p(packed.data_ptr()), C.c_void_p(xs.data_ptr()),
+                                    C.c_void_p(ts.data_ptr()), C.c_int64(rows), C.c_void_p(ws.data_ptr() + off),
+                                    C.c_int64(need), C.c_void_p(loss.data_ptr()),
+                                    _lib.void_ptr_array([a.data_ptr() for a, _ in grads]),
+                                    _lib.void_ptr_array([b.data_ptr() for _, b in grads]),
+                                    C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        _lib.check(rc, "train step")
+        torch.cuda.synchronize()
+        assert bool((ws[:off] == 0x5A).all()) and bool((ws[off + need:] == 0x5A).all()), "written outside the workspace"
+        sloss, sgrads = _run(lib, p, packed, xs, ts, static=True)
+        assert torch.isfinite(sloss) and torch.equal(sloss, loss.cpu())
+        for (a, b), (c, d) in zip(sgrads, grads):
+            assert torch.equal(a, c.cpu()) and torch.equal(b, d.cpu())
