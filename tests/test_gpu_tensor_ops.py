@@ -65,12 +65,17 @@ def test_linear_tensor_op_fp32_matches_oracle(shape):
 
 
 @pytest.mark.parametrize("rows,inf,outf", [
-    (16390, 48, 1020), (4100, 80, 1000), (2050, 72, 1000), (4099, 64, 252), (70, 136, 36),  # each block tile, ragged
-    (1, 8, 4), (33, 64, 16), (257, 72, 260),   # one row; exactly one K step; one row past a tile
+    # ragged; the tile the rule takes on 256 CUs, fp16 and fp32 (S: linear_stream_kernel)
+    (16380, 200, 1020),                       # 256 x 256 both, four K steps and seven
+    (8190, 72, 1020), (4090, 72, 500),        # 128 x 128 both; 128 x 64 both
+    (9000, 72, 500),                          # 64 x 64 both
+    (16390, 48, 1020), (4100, 80, 1000), (2050, 72, 1000), (4099, 64, 252), (70, 136, 36),
+    #  128 x 128, S     64 x 64 both       128 x 128, 64 x 32  128 x 64, 64 x 32  64 x 32 both
+    (1, 8, 4), (33, 64, 16), (257, 72, 260),   # one row; exactly one K step; one row past a tile: 64 x 32 both
 ])
 @pytest.mark.parametrize("kind", ["f32", "f16_w32", "f16_w16", "f16_tiled", "f16_tiled_odd"])
 def test_linear_op_tiles(rows, inf, outf, kind):
-    """Every block tile and weight kind of the linear kernel at ragged sizes, within twice the bound of any fp32
+    """Every block tile and weight kind of the linear kernels at ragged sizes, within twice the bound of any fp32
     summation order; nothing past the last row is written.  f16_tiled_odd: a tile copy off 16-byte alignment."""
     tiled = kind.startswith("f16_tiled")
     if tiled:

@@ -177,7 +177,7 @@ def test_c5_full_config_against_cpu_restatement():
            "C5 full size vs the CPU restatement")
 
 
-@pytest.mark.parametrize("n", [1, 33, 1000, 20011])  # one point; a tile and a point; ragged; several tiles per wave
+@pytest.mark.parametrize("n", [1, 33, 1000, 20011])  # one point; a tile and a point; ragged; a tile for most waves
 @pytest.mark.parametrize("dims", [
     [16, 32, 8], [48] + [32] * 5 + [16], [64] + [32] * 4 + [8],               # 32 wide, 1 to 5 hidden layers
     [16, 64, 16], [32] + [64] * 4 + [16], [48, 64, 64, 8], [64] + [64] * 4 + [8],  # 64 wide, 1 to 4; 1 to 4 input chunks
@@ -267,3 +267,23 @@ def test_narrow_chains_keep_non_finite_values_apart(dims, n, where, value):
             assert (np.isfinite(a) == finite).all(), f"layer {l} {what}: {(np.isfinite(a) != finite).sum()} entries"
             err = np.linalg.norm(a[finite] - b[finite])
             assert err <= 1e-2 * np.linalg.norm(b[finite]), f"layer {l} {what}: {err}"
+
+
+@pytest.mark.parametrize("dims,n", [
+    ([16, 32, 8], 140011), ([48] + [32] * 5 + [16], 140011), ([64] + [32] * 4 + [8], 200001),  # 2,048 waves: 2 to 4 tiles each
+    ([16, 64, 16], 70001), ([48, 64, 64, 8], 70001), ([32] + [64] * 3 + [16], 140011), ([64] + [64] * 4 + [8], 70001),  # 1,024
+])
+def test_narrow_chains_over_several_tiles(dims, n):
+    """The kernel's tile loop past its first turn: the prefetched inputs, the gradients, db and loss carried over tiles,
+    ragged ends, against the oracle at the step's bars."""
+    g = torch.Generator().manual_seed(n)
+    layers = []
+    for i in range(len(dims) - 1):
+        lim = (6.0 / dims[i]) ** 0.5
+        layers.append((((torch.rand(dims[i + 1], dims[i], generator=g) * 2 - 1) * lim).half().float(),
+                       torch.randn(dims[i + 1], generator=g) * 0.1))
+    x = torch.randn(n, dims[0], generator=g).half()
+    t = torch.randn(n, dims[-1], generator=g)
+    loss, grads = rdv.mse_backward(_chain(layers), x.cuda(), t.cuda())
+    ref_loss, ref_grads = T.mse_grads(x.float().numpy(), [(w.numpy(), b.numpy()) for w, b in layers], t.numpy())
+    _check(loss.item(), grads, ref_loss, ref_grads, f"{dims} n={n}")
