@@ -14,8 +14,8 @@
 // at dispatch, like Small and Mine), fp16 [out, in] (Simple's pre-cast copy) or
 // fp16 [out/16][in/16][16 k][16 n] tiles (Fast's pre-tiled copy, nn.py:472-490).
 //
-// linear_gemm_kernel (below) serves most shapes, linear_stream_kernel large fp32
-// products over few columns; relu_op_kernel streams.
+// linear_gemm_kernel (below) serves most shapes, linear_stream_kernel large products
+// over few columns; relu_op_kernel streams.
 #include <algorithm>
 
 #include "rdv_common.h"
@@ -321,32 +321,34 @@ int launch_linear_gemm_t(const LinearGemmArgs& a0, hipStream_t stream) {
   return RDV_OK;
 }
 
-// -------------------------------------------------- few columns, many rows (fp32)
+// --------------------------------------------------------- few columns, many rows
 // A persistent block of 4 waves owns up to 128 outputs: it stages their weights and
-// biases in LDS once, as the A fragments of v_mfma_f32_16x16x4f32 (slot (t, c, lane):
-// W[o0 + 16 t + lane % 16][16 c + 4 (lane / 16) ..]), then its waves walk 32-row tiles
+// biases in LDS once, as A fragments (slot (t, c, lane): W[o0 + 16 t + lane % 16][16 c +
+// 4 (lane / 16) ..] for v_mfma_f32_16x16x4f32, [32 c + 8 (lane / 16) ..] for
+// v_mfma_f32_16x16x32_f16), then its waves walk 32-row tiles
 // with a grid stride and no barrier, the next tile's x loaded (16 bytes a lane)
 // while this one is computed.  The products and their order are linear_gemm_kernel's.
 //
-// linear_gemm_kernel stages whole steps of 32 columns and its blocks load, compute and
+// linear_gemm_kernel stages whole steps of 32 (fp16: 64) columns and its blocks load, compute and
 // store in turn; with one or two steps there is little to overlap, and up to half of
 // it is padding.  Bound: HBM.  Measured, gemm and this kernel: 262,144 x 8 -> 128 37.7 and
 // 24.7 us, 65,536 x 48 -> 512 56 and 42, 65,536 x 16 -> 1024 76 and 47, 4,194,304 x 8 -> 4 111
-// and 58.
+// and 58; fp16 65,536 x 16 -> 1024 60 and 48, 4,194,304 x 8 -> 16 124 and 78.
 constexpr int kLsThreads = 256, kLsWaves = 4, kLsOutputs = 128, kLsRows = 32;  // rows per wave and tile
 
 struct LinearStreamArgs {
   const float* x;
-  const float* w;
+  const void* w;
   const float* bias;
   float* y;
   int64_t rows, tasks;  // tasks: tiles of kLsWaves * kLsRows rows
-  int in, out, relu;
+  int in, out, wkind, relu;
   int ob, n_ob;         // outputs per block (a multiple of 16), blocks of outputs
 };
 
-template <int NKC, int G>  // chunks of 16 columns, tiles of 16 outputs stored together
+template <bool F16, int NKC, int G>  // chunks of 32 (fp16) or 16 columns, tiles of 16 outputs stored together
 __global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamArgs a) {
+  constexpr int KC = F16 ? 32 : 16, PV = F16 ? 2 : 1;  // columns per chunk, 16-byte loads per lane and chunk
   extern __shared__ f32x4 lo_smem[];
   const int nt = a.ob / 16;
   f32x4* const sw = lo_smem;                     // [nt][NKC][64]
@@ -359,13 +361,25 @@ __global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamA
   const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int s = threadIdx.x; s < nt * NKC * 64; s += kLsThreads) {
     const int o = o0 + 16 * (s / (NKC * 64)) + (s & 15);
-    const int k = 16 * ((s >> 6) % NKC) + 4 * ((s & 63) >> 4);
-    sw[s] = o < a.out && k < a.in ? *reinterpret_cast<const f32x4*>(a.w + int64_t(o) * a.in + k) : zero4;
+    const int k = KC * ((s >> 6) % NKC) + KC / 4 * ((s & 63) >> 4);
+    f32x4 v = zero4;
+    if (o < a.out && k < a.in) {
+      const int64_t e = int64_t(o) * a.in + k;
+      if (!F16) {
+        v = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.w) + e);
+      } else if (a.wkind == RDV_WKIND_F32) {
+        const f32x4* src = reinterpret_cast<const f32x4*>(static_cast<const float*>(a.w) + e);
+        v = __builtin_bit_cast(f32x4, to_half8(src[0], src[1]));
+      } else {
+        v = *reinterpret_cast<const f32x4*>(static_cast<const half_t*>(a.w) + e);
+      }
+    }
+    sw[s] = v;
   }
   for (int i = threadIdx.x; i < a.ob; i += kLsThreads) reinterpret_cast<float*>(sb)[i] = o0 + i < a.out ? a.bias[o0 + i] : 0.0f;
   __syncthreads();
 
-  f32x4 raw[2][NKC], xf[2][NKC];
+  f32x4 raw[2][NKC][PV], xf[2][NKC];
   // rows clamped into range (their results are not stored), columns past `in` to
   // column 0 (zeroed on use): every load is in bounds
   auto load = [&](int64_t task) {
@@ -374,7 +388,11 @@ __global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamA
       const int64_t row = (task * kLsWaves + wave) * kLsRows + 16 * h + r;
       const float* xr = a.x + (row < a.rows ? row : a.rows - 1) * a.in;
 #pragma unroll
-      for (int c = 0; c < NKC; ++c) raw[h][c] = *reinterpret_cast<const f32x4*>(xr + (16 * c + 4 * q < a.in ? 16 * c + 4 * q : 0));
+      for (int c = 0; c < NKC; ++c) {
+        const int k = KC * c + KC / 4 * q;
+#pragma unroll
+        for (int v = 0; v < PV; ++v) raw[h][c][v] = reinterpret_cast<const f32x4*>(xr + (k < a.in ? k : 0))[v];
+      }
     }
   };
   int64_t task = blockIdx.x / unsigned(a.n_ob);
@@ -383,7 +401,11 @@ __global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamA
 #pragma unroll
     for (int c = 0; c < NKC; ++c)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) xf[h][c] = 16 * c + 4 * q < a.in ? raw[h][c] : zero4;
+      for (int h = 0; h < 2; ++h) {
+        f32x4 v = raw[h][c][0];
+        if constexpr (F16) v = __builtin_bit_cast(f32x4, to_half8(raw[h][c][0], raw[h][c][PV - 1]));
+        xf[h][c] = KC * c + KC / 4 * q < a.in ? v : zero4;
+      }
     load(task + stride < a.tasks ? task + stride : a.tasks - 1);
     const int64_t row0 = (task * kLsWaves + wave) * kLsRows + r;
     float* const y0 = a.y + row0 * a.out + o0 + 4 * q;
@@ -399,10 +421,17 @@ __global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamA
 #pragma unroll
         for (int c = 0; c < NKC; ++c) {
           const f32x4 wv = sw[(t * NKC + c) * 64 + lane];
+          if constexpr (F16) {
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
+            for (int h = 0; h < 2; ++h)
+              acc[u][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, wv), __builtin_bit_cast(half8, xf[h][c]),
+                                                                 acc[u][h], 0, 0, 0);
+          } else {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) acc[u][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[k], xf[h][c][k], acc[u][h], 0, 0, 0);
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+              for (int h = 0; h < 2; ++h) acc[u][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[k], xf[h][c][k], acc[u][h], 0, 0, 0);
+          }
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -425,22 +454,22 @@ __global__ __launch_bounds__(kLsThreads) void linear_stream_kernel(LinearStreamA
   }
 }
 
-template <int NKC, int G>
+template <bool F16, int NKC, int G>
 int launch_linear_stream_t(const LinearStreamArgs& a, int cu, hipStream_t stream) {
   const size_t lds = size_t(a.ob / 16) * NKC * 1024 + size_t(a.ob) * 4;  // at most 32.5 KiB
   int occ = 0;
-  RDV_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, linear_stream_kernel<NKC, G>, kLsThreads, lds));
+  RDV_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, linear_stream_kernel<F16, NKC, G>, kLsThreads, lds));
   const int64_t slots = int64_t(cu) * std::max(occ, 1);
   const int64_t groups = std::max<int64_t>(1, std::min<int64_t>(a.tasks, (slots + a.n_ob - 1) / a.n_ob));
-  linear_stream_kernel<NKC, G><<<dim3(unsigned(groups * a.n_ob)), dim3(kLsThreads), lds, stream>>>(a);
+  linear_stream_kernel<F16, NKC, G><<<dim3(unsigned(groups * a.n_ob)), dim3(kLsThreads), lds, stream>>>(a);
   RDV_HIP_TRY(hipGetLastError());
   return RDV_OK;
 }
 
-template <int NKC>
+template <bool F16, int NKC>
 int launch_linear_stream(const LinearStreamArgs& a, int cu, hipStream_t stream) {
-  if (a.ob == kLsOutputs && a.rows * a.out >= int64_t(1) << 27) return launch_linear_stream_t<NKC, 8>(a, cu, stream);
-  return launch_linear_stream_t<NKC, 2>(a, cu, stream);
+  if (a.ob == kLsOutputs && a.rows * a.out >= int64_t(1) << 27) return launch_linear_stream_t<F16, NKC, 8>(a, cu, stream);
+  return launch_linear_stream_t<F16, NKC, 2>(a, cu, stream);
 }
 
 __global__ __launch_bounds__(256) void relu_op_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t n) {
@@ -509,24 +538,29 @@ int launch_linear_op(const rdv_linear_op_desc& d, const float* x, const void* w,
   DeviceInfo dev;
   if (int rc = device_info(&dev)) return rc;
   const bool f16 = d.precision == RDV_PREC_F16;
-  if (!f16 && d.in_features <= 64) {
+  if (d.in_features <= (f16 ? 16 : 64) && d.wkind != RDV_WKIND_F16_TILED16) {
     // linear_stream_kernel where its blocks fill the chip, so many per CU that it is the
-    // faster of the two (us, linear_gemm_kernel and this one, just below and at the line):
-    // up to 16 columns 2 (32,768 x 8 -> 128, 1 per CU, 7.7 and 7.0; 65,536 x 8 -> 128 12.3 and
-    // 9.7), to 32 4 (65,536 x 32 -> 128, 2, 12.8 and 12.9; 65,536 x 24 -> 256 21.5 and 19.6),
-    // to 48 2 (32,768 x 48 -> 128, 1, 10.4 and 10.5; 65,536 x 40 -> 128 17.9 and 15.8), to 64 8
-    // (32,768 x 64 -> 512, 4, 29.4 and 30.9; 65,536 x 64 -> 512 55.1 and 51.5).
-    LinearStreamArgs a = {x, static_cast<const float*>(w), bias, y, d.rows, 0, d.in_features, d.out_features, d.relu ? 1 : 0, 0, 0};
+    // faster of the two (us, linear_gemm_kernel and this one, just below and at the line).
+    // fp32: up to 16 columns 2 (32,768 x 8 -> 128, 1 per CU, 7.7 and 7.0; 65,536 x 8 -> 128
+    // 12.3 and 9.7), to 32 4 (65,536 x 32 -> 128, 2, 12.8 and 12.9; 65,536 x 24 -> 256 21.5
+    // and 19.6), to 48 2 (32,768 x 48 -> 128, 1, 10.4 and 10.5; 65,536 x 40 -> 128 17.9 and
+    // 15.8), to 64 8 (32,768 x 64 -> 512, 4, 29.4 and 30.9; 65,536 x 64 -> 512 55.1 and 51.5).
+    // fp16: up to 16 columns 4 (65,536 x 16 -> 128, 2, 9.8 and 9.7; 65,536 x 16 -> 256 16.9 and
+    // 14.6), and past 2^18 rows, where the gemm's larger tiles write better, 32 outputs
+    // (2^20 x 8 -> 32 32 and 27, 2^20 x 8 -> 64 82 and 95).  fp16 tiles, which the gemm moves by
+    // DMA, are within 9% either way.
+    LinearStreamArgs a = {x, w, bias, y, d.rows, 0, d.in_features, d.out_features, d.wkind, d.relu ? 1 : 0, 0, 0};
     a.tasks = (d.rows + kLsWaves * kLsRows - 1) / (kLsWaves * kLsRows);
     a.ob = std::min(kLsOutputs, (d.out_features + 15) / 16 * 16);
     a.n_ob = (d.out_features + a.ob - 1) / a.ob;
     const int chunks = (d.in_features + 15) / 16;
-    const int per_cu = chunks == 4 ? 8 : chunks == 2 ? 4 : 2;
-    if (a.tasks * a.n_ob >= int64_t(per_cu) * dev.cu_count) {
-      if (chunks == 1) return launch_linear_stream<1>(a, dev.cu_count, stream);
-      if (chunks == 2) return launch_linear_stream<2>(a, dev.cu_count, stream);
-      if (chunks == 3) return launch_linear_stream<3>(a, dev.cu_count, stream);
-      return launch_linear_stream<4>(a, dev.cu_count, stream);
+    const int per_cu = f16 ? 4 : chunks == 4 ? 8 : chunks == 2 ? 4 : 2;
+    if (a.tasks * a.n_ob >= int64_t(per_cu) * dev.cu_count && (!f16 || d.rows <= 1 << 18 || d.out_features <= 32)) {
+      if (f16) return launch_linear_stream<true, 1>(a, dev.cu_count, stream);
+      if (chunks == 1) return launch_linear_stream<false, 1>(a, dev.cu_count, stream);
+      if (chunks == 2) return launch_linear_stream<false, 2>(a, dev.cu_count, stream);
+      if (chunks == 3) return launch_linear_stream<false, 3>(a, dev.cu_count, stream);
+      return launch_linear_stream<false, 4>(a, dev.cu_count, stream);
     }
   }
   // The tile whose busiest CU has the least work: tiles per CU, rounded up, times

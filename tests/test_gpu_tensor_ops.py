@@ -416,16 +416,21 @@ def test_more_threads_than_one_launch_takes(rows, inf, outf):
     (65599, 56, 512), (262145, 64, 20), ((1 << 20) + 1, 16, 128),  # the last: y of 2^27 elements and more
 ])
 @pytest.mark.parametrize("relu", [False, True])
-def test_linear_op_few_columns(rows, inf, outf, relu):
-    """fp32 products of up to 64 columns at row counts that take the streaming kernel, ragged in every dimension, within
+@pytest.mark.parametrize("kind", ["f32", "f16_w32", "f16_w16"])  # fp16: the streaming kernel up to 16 columns
+def test_linear_op_few_columns(rows, inf, outf, relu, kind):
+    """Products of up to 64 columns at row counts that take the streaming kernel, ragged in every dimension, within
     twice the bound of any fp32 summation order; nothing past the last row is written."""
     g = torch.Generator(device="cuda").manual_seed(rows + inf)
     x = torch.randn(rows, inf, generator=g, device="cuda")
     W = torch.randn(outf, inf, generator=g, device="cuda") / inf ** 0.5
     b = torch.randn(outf, generator=g, device="cuda")
     y = torch.full(((rows + 2) * outf,), 12345.0, device="cuda")
-    assert _raw_linear(x, W, b, y, rows, inf, outf, _lib.PREC_F32, _lib.WKIND_F32, relu) == 0, _lib.last_error()
+    f16 = kind != "f32"
+    w, wk = (W.half(), _lib.WKIND_F16) if kind == "f16_w16" else (W, _lib.WKIND_F32)
+    assert _raw_linear(x, w, b, y, rows, inf, outf, _lib.PREC_F16 if f16 else _lib.PREC_F32, wk, relu) == 0, _lib.last_error()
     assert bool((y[rows * outf:] == 12345.0).all()), "kernel wrote past the last row"
+    if f16:
+        x, W = x.half().float(), W.half().float()
     u, k = 2.0 ** -24, inf + 2
     for r in range(0, rows, 1 << 18):
         xr = x[r:r + (1 << 18)].double()
